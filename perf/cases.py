@@ -226,6 +226,8 @@ def prepare(case, seed):
         s["c"], s["cs"] = torch.empty(m, k // 2, dtype=torch.uint8, device="cuda"), torch.empty(m, k // 32, dtype=torch.uint8, device="cuda")
         s["cst"] = torch.zeros(rfp4.mx4_scales_tiled_bytes(m, k), dtype=torch.uint8, device="cuda")
         s["y"] = torch.empty(m, n, **f32)
+    # the handles that a program holds: its stream and its buffers' addresses
+    s["stream"], s["ptr"] = _stream(), {name: t.data_ptr() for name, t in s.items() if isinstance(t, torch.Tensor)}
     return s
 
 
@@ -242,8 +244,7 @@ def run(s):
     if op == "generate":
         ids = s["eng"].generate(s["prompt"], s["ctx"], s["new"])
         return {"ids": ids, "logits": s["eng"].logits(), "k": s["written"][0], "v": s["written"][1]}
-    c, st = s["case"], _stream()
-    p = {k: v.data_ptr() for k, v in s.items() if isinstance(v, torch.Tensor)}
+    c, st, p = s["case"], s["stream"], s["ptr"]
     if op == "gemv":
         (rfp4.fp4_gemv if c["scale"] == "f32" else rfp4.mx4_gemv)(st, c["n"], c["k"], p["w"], p["ws"], p["x"], p["y"])
     elif op == "mlp":
