@@ -115,7 +115,7 @@ int mx4_gemv(rfp4_stream_t stream, uint32_t n, uint32_t k, const uint8_t *codes,
  *                     reference's tie rule (fp4_gemv lm_head + argmax, :533-534);
  *                     workspace: at least mx4_gemv_argmax_workspace(n) =
  *                     round_up(n, 8) + 64 bytes, 8-byte aligned (one 8-byte key
- *                     per workgroup, then a 16-byte cursor).  The library cannot
+ *                     per workgroup of at least 8 rows).  The library cannot
  *                     see the caller's allocation: a smaller buffer is written
  *                     out of bounds, so size it with that function. */
 /* rmsnorm + fp4_gemv (llama_run/src/main.rs:513-514 fused): y = W.(x*rms*w_norm),

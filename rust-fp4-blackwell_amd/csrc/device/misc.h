@@ -69,12 +69,20 @@ RFP4_DEV void argmax_body(const ArgmaxArgs &a)
     }
 }
 
-// ---------------------------------------------------------------- end of decode step
-RFP4_DEV void step_body(const StepArgs &a)
+// The largest of n per-workgroup keys (one workgroup of 1024 threads): each
+// thread's loads of four keys issued together, then the wave and workgroup
+// reductions.  Thread 0 returns the maximum.
+RFP4_DEV unsigned long long keys_max(const unsigned long long *keys, uint32_t n)
 {
     __shared__ unsigned long long red[16];
     unsigned long long best = 0ull;
-    for (uint32_t i = threadIdx.x; i < a.n_best; i += blockDim.x) best = a.best[i] > best ? a.best[i] : best;
+    for (uint32_t i0 = threadIdx.x; i0 < n; i0 += 4u * blockDim.x) {
+        unsigned long long v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = keys[min(i0 + (uint32_t)j * blockDim.x, n - 1u)];
+#pragma unroll
+        for (int j = 0; j < 4; j++) best = v[j] > best ? v[j] : best;
+    }
     for (int off = 32; off >= 1; off >>= 1) {
         unsigned long long o = __shfl_xor(best, off, 64);
         best = o > best ? o : best;
@@ -82,10 +90,28 @@ RFP4_DEV void step_body(const StepArgs &a)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     if (lane == 0) red[wave] = best;
     __syncthreads();
+    unsigned long long b = red[0];
+    for (int w = 1; w < nw; w++) b = red[w] > b ? red[w] : b;
+    return b;
+}
+
+// The token of an argmax GEMV's keys (ArgmaxKeysArgs): where no decode cursor
+// moves (mx4_gemv_argmax, the batched prefill's last row).  Latency bound
+// (4008 keys of a 128256-row head: 5.3 us in the trace, one launch instead of
+// the 4.6 + 4.5 us of clearing a scratch cursor and running the step kernel;
+// the prefill ran the one-workgroup argmax over all logits, 49.7 us).
+RFP4_DEV void argmax_keys_body(const ArgmaxKeysArgs &a)
+{
+    const unsigned long long b = keys_max(a.best, a.n_best);
+    if (threadIdx.x == 0) *a.out = 0xFFFFFFFFu - (uint32_t)(b & 0xFFFFFFFFull);
+}
+
+// ---------------------------------------------------------------- end of decode step
+RFP4_DEV void step_body(const StepArgs &a)
+{
+    const unsigned long long b = keys_max(a.best, a.n_best);
     __shared__ uint32_t s_next;
     if (threadIdx.x == 0) {
-        unsigned long long b = red[0];
-        for (int w = 1; w < nw; w++) b = red[w] > b ? red[w] : b;
         uint32_t tok = 0xFFFFFFFFu - (uint32_t)(b & 0xFFFFFFFFull);
         StepState st = *a.state;
         *a.last_tok = tok;

@@ -11,14 +11,28 @@
 
 #define RQ_U 4 // elements per thread whose loads are issued together in the row kernels
 
-// grid (rows): y[r] = widen(embed[ids[r]])  (llama_run/src/main.rs:509-510)
+// grid (rows, parts): y[r] = widen(embed[ids[r]])  (llama_run/src/main.rs:509-510).
+// Bound by the latency of the gather: one 16-byte load and two float4 stores
+// per thread (k is a multiple of 256 here, so rows start 16-byte aligned), a
+// workgroup per 2048 elements of a row, so that a row takes one round trip
+// (one element per thread and trip before: 700 rows x 4096 12.9 us, now 9.3).
 RFP4_DEV void embed_rows_body(const RowsArgs &a)
 {
-    const uint32_t r = blockIdx.x;
+    const uint32_t r = blockIdx.x, i = blockIdx.y * blockDim.x + threadIdx.x;
+    if (i >= a.k / 8u) return;
     uint32_t tok = a.ids[r];
     if (tok >= a.vocab) tok = 0;
-    const uint16_t *row = a.embed + (size_t)tok * a.k;
-    for (uint32_t i = threadIdx.x; i < a.k; i += blockDim.x) a.y[(size_t)r * a.k + i] = half_bits_to_f32(row[i], a.bf16 != 0);
+    const u32x4 w = ((const u32x4 *)(a.embed + (size_t)tok * a.k))[i];
+    const bool bf16 = a.bf16 != 0;
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        v[2 * j] = half_bits_to_f32(w[j] & 0xFFFFu, bf16);
+        v[2 * j + 1] = half_bits_to_f32(w[j] >> 16, bf16);
+    }
+    float4 *y = (float4 *)(a.y + (size_t)r * a.k) + 2u * i;
+    y[0] = make_float4(v[0], v[1], v[2], v[3]);
+    y[1] = make_float4(v[4], v[5], v[6], v[7]);
 }
 
 // grid (rows): RMSNorm of row r with fp16 weights, in the order of

@@ -457,7 +457,7 @@ static int enqueue_prefill(llama_engine *e, uint32_t n, uint32_t pos0)
     RowsArgs ea{};
     ea.ids = e->pf_ids; ea.embed = e->embed; ea.y = e->pf_x; ea.rows = n; ea.k = c.dim; ea.vocab = c.vocab;
     ea.bf16 = e->embed_bf16;
-    if ((rc = launch("rfp4_embed_rows", dim3(n), dim3(256), s, &ea))) return rc;
+    if ((rc = launch("rfp4_embed_rows", dim3(n, (c.dim + 2047u) / 2048u), dim3(256), s, &ea))) return rc;
     // test hook: stop after stage `stop` (-1: the embedding; 10 * layer + s: stage s of that layer)
     const int stop = prefill_stop();
     if (stop == -1) return kPrefillStopped;
@@ -571,13 +571,14 @@ static int enqueue_prefill(llama_engine *e, uint32_t n, uint32_t pos0)
         if (l + 1 == c.n_layers && !down_in_x && (rc = residual(s, n * c.dim, e->pf_c, e->pf_x))) return rc;
     }
 #undef RFP4_PF_STAGE
-    // last row: the decode step's final norm + LM head, then argmax
-    rc = hip_check(hipMemcpyAsync(e->x, e->pf_x + (size_t)(n - 1) * c.dim, c.dim * sizeof(float),
-                                  hipMemcpyDeviceToDevice, s), "hipMemcpyAsync(prefill row)");
-    GemvArgs la{e->lm_c, e->lm_s, e->x, e->logits, nullptr, e->norm_final, c.vocab, c.dim, 0, c.eps};
-    if (!rc) rc = gemv_launch(e->sname, RFP4_EPI_STORE, la, s);
-    if (!rc) rc = argmax(s, c.vocab, e->logits, e->last_tok);
-    return rc;
+    // last row, read where it lies: the decode step's final norm, LM head and
+    // per-workgroup argmax keys, then their reduction.  (The stand-alone
+    // argmax over 128256 logits, one workgroup, took 49.7 us here; the copy of
+    // the row into e->x 3-5 us.)
+    GemvArgs la{e->lm_c, e->lm_s, e->pf_x + (size_t)(n - 1) * c.dim, e->logits, e->best, e->norm_final, c.vocab, c.dim, 0,
+                c.eps};
+    if ((rc = gemv_launch_v(e->sname, RFP4_EPI_ARGMAX, la, s, e->gv[GV_LM]))) return rc;
+    return argmax_keys_launch(e->best, e->n_best, e->last_tok, s);
 }
 
 static uint32_t splits_at(const llama_engine *e, int64_t pos)

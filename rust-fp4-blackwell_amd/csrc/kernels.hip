@@ -167,6 +167,7 @@ K256 void rfp4_copy_into_f16(CopyArgs a) { copy_into_body<1>(a); }
 K256 void rfp4_swiglu(EltwiseArgs a) { swiglu_body(a); }
 K256 void rfp4_residual(EltwiseArgs a) { residual_body(a); }
 K1024 void rfp4_argmax(ArgmaxArgs a) { argmax_body(a); }
+K1024 void rfp4_argmax_keys(ArgmaxKeysArgs a) { argmax_keys_body(a); }
 K1024 void rfp4_step(StepArgs a) { step_body(a); }
 K256 void rfp4_synth_weight(SynthWeightArgs a) { synth_weight_body(a); }
 K256 void rfp4_synth_f16(SynthF16Args a) { synth_f16_body(a); }

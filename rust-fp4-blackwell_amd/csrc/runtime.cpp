@@ -885,8 +885,21 @@ int mx4_gemv_swiglu(rfp4_stream_t stream, uint32_t n, uint32_t k, uint32_t pair_
 
 size_t mx4_gemv_argmax_workspace(uint32_t n) { return ((size_t)n + 7u) / 8u * 8u + 64u; /* >= one key per 8 rows */ }
 
-// The per-workgroup keys of an argmax GEMV, then the step kernel's reduction
-// on a scratch cursor after the keys (ids_cap = 0: no ids are written).
+} // extern "C"
+
+namespace rfp4 {
+
+int argmax_keys_launch(const unsigned long long *best, uint32_t n_best, uint32_t *out, hipStream_t s)
+{
+    ArgmaxKeysArgs ka{best, out, n_best, 0};
+    return launch("rfp4_argmax_keys", dim3(1), dim3(1024), s, &ka);
+}
+
+} // namespace rfp4
+
+extern "C" {
+
+// The per-workgroup keys of an argmax GEMV, then their reduction.
 static int gemv_argmax_launch(hipStream_t s, const char *sname, const GemvArgs &args, void *workspace,
                               uint32_t *best_token)
 {
@@ -897,11 +910,7 @@ static int gemv_argmax_launch(hipStream_t s, const char *sname, const GemvArgs &
                          mx4_gemv_argmax_workspace(args.n));
     int rc = gemv_launch_v(sname, RFP4_EPI_ARGMAX, args, s, v);
     if (rc) return rc;
-    StepState *st = (StepState *)((char *)workspace + (size_t)nb * 8u);
-    rc = fill_words((uint32_t *)st, sizeof(StepState) / 4, 0u, s);
-    if (rc) return rc;
-    StepArgs sa{args.best, st, nullptr, best_token, nb, 0};
-    return launch("rfp4_step", dim3(1), dim3(1024), s, &sa);
+    return argmax_keys_launch((const unsigned long long *)workspace, nb, best_token, s);
 }
 
 int mx4_gemv_argmax(rfp4_stream_t stream, uint32_t n, uint32_t k, const uint8_t *codes, const uint8_t *scales,

@@ -63,6 +63,13 @@ typedef struct ArgmaxArgs {
     uint32_t n, pad;
 } ArgmaxArgs;
 
+// The token of the largest of an argmax GEMV's per-workgroup keys.
+typedef struct ArgmaxKeysArgs {
+    const unsigned long long *best;
+    uint32_t *out;
+    uint32_t n_best, pad;
+} ArgmaxKeysArgs;
+
 // Split-K flash-decode attention.
 typedef struct AttnArgs {
     const float *q;       // [n_heads][head_dim]
