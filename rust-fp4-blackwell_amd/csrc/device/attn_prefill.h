@@ -5,13 +5,14 @@
 // (llama_run/src/main.rs:148-242 applied row by row), with the prompt's own
 // rows already appended to the fp16 caches.
 //
-// Grid (query tiles, n_kv_heads).  A workgroup of NW waves takes BQ =
-// max(16, 16 NW / GT) prompt rows and every query head of one KV head (GT
-// heads, G <= GT real), i.e. NT = (BQ/16) * GT tiles of 16 (row, head) pairs,
-// MT = NT / NW per wave, and walks the keys 0 .. last
-// row's position in blocks of 64 keys (head dim 64) or 32 (128): K rows staged in LDS as loaded, V rows
-// staged transposed (dimension-major), as v_mfma_f32_16x16x32_f16 operands,
-// every product transposed so that the scores' accumulator is the next
+// A workgroup of NW waves per key group takes BQ = max(16, 16 NW / GT) prompt
+// rows and every query head of one KV head (GT heads, G <= GT real), i.e. NT =
+// (BQ/16) * GT tiles of 16 (row, head) pairs, MT = NT / NW per wave, and walks
+// the keys 0 .. last row's position in blocks of 64 keys (head dim 64) or 32
+// (128).  K and V rows are staged in LDS by DMA as they lie in the cache
+// (chunks XOR-swizzled, no bank conflicts: SQ_LDS_BANK_CONFLICT 0); V^T
+// operands come out of the row-major rows through the transposing LDS read.
+// Every product is transposed so that the scores' accumulator is the next
 // product's operand as it lies in the registers:
 //   S^T (32 x 16) = K (32 x HD) . Q^T         -- B = q as two fp16 terms
 //   online softmax per row (base 2, f32)      -- a row lives in the 4 lanes
@@ -20,8 +21,18 @@
 // Lane (q4 = l / 16, row l % 16) holds the scores of keys 4 q4 .. +3 and
 // 16 + 4 q4 .. +3 of each 32-key half of a block, which are the 8 K values
 // of its P^T operand for that half; the V^T operand takes the same 8 keys of
-// each dimension (two 8-byte reads of the transposed V rows), so P never
-// leaves the registers.
+// each dimension (two transposing reads), so P never leaves the registers.
+//
+// What bounds it: matrix and vector instructions of 4 waves per SIMD.  At 2048
+// rows after 2048 keys of the 8B heads (206 GFLOP with the hi + lo terms, 191
+// us) the matrix cores are busy 57 % of the cycles and the vector ALU about as
+// much; LDS reads take 29 %.  Staging through registers (V transposed by 2-byte
+// LDS writes, two register sets of loads) needed 141 registers, so a CU held
+// one workgroup of 8 waves: 1531 rows after 517 keys 146 us, by DMA 93 us, with
+// two key groups of 4 waves 81 us, with the rarely raised maximum, uniform DMA
+// bases and two interleaved score chains 75 us (267 -> 191 us at 2048 + 2048,
+// 33 -> 20.5 us at 700 rows).  At most 128 registers keep 4 waves per SIMD.
+//
 // q and p enter as hi + lo (hi = fp16(x), lo = fp16(x - hi): about 2^-22
 // relative, two MFMAs per product; K and V are fp16 already), products exact
 // and f32 accumulation, so the output matches the f32 decode kernel's to
@@ -30,13 +41,74 @@
 // logits by percent.  Operand
 // layout (pinned by the fp16 layout test): lane l holds A row / B column
 // l % 16 and K = 8 (l / 16) .. +7; accumulator r of lane l is D[4 (l/16) + r][l % 16].
-// The next two blocks' K/V loads are in flight while the current block computes.
 #pragma once
 #include "common.h"
 #include "misc.h"
 
-#define PF_KPAD 8  // fp16 padding of a staged K row (16 consecutive rows -> 16 distinct bank groups)
-#define PF_TPAD 8  // fp16 padding of a transposed V row
+typedef __attribute__((address_space(3))) uint8_t pf_lds_u8;
+typedef __attribute__((address_space(1))) void pf_glb_void;
+#define PF_VMCNT(V) (((V) & 0xFu) | (((V) >> 4) << 14) | (0x7u << 4) | (0xFu << 8)) // s_waitcnt vmcnt(V)
+
+// Chunk swizzles of the staged rows (the physical chunk of logical chunk q of
+// row r is q ^ swizzle(r)).  K rows are read 16 at a time, one chunk of each:
+// 16 rows of 256 bytes (HD 128), or 16 of 128 (HD 64, two rows per 256-byte
+// bank line), fall on 16 distinct chunks of a bank line.  V rows are read 8
+// at a time (by half a wave), 32 bytes of each: the swizzle moves pairs of
+// chunks, so 8 rows cover a bank line once.
+template <int HD>
+RFP4_DEV uint32_t pf_kswz(uint32_t r)
+{
+    return HD == 128 ? r & 15u : (r ^ ((r >> 3) & 1u)) & 7u;
+}
+template <int HD>
+RFP4_DEV uint32_t pf_vswz(uint32_t r)
+{
+    return HD == 128 ? (r & 7u) << 1 : ((r >> 1) & 3u) << 1;
+}
+
+// LDS reads in inline asm: the compiler treats every LDS read after an LDS DMA
+// as a possible alias of it and would wait for every DMA in flight.  Each asm
+// waits for its own reads, so no register of a read in flight is ever visible
+// outside it.
+// pf_read_k: four K operands, rows 16 h + l16 and chunk 4 k + q4 of the block
+// (a step of k is an XOR of 4 chunks on the address, a step of h 16 rows): HD
+// 128 k = k0, k0 + 1 of both 16-key quarters (ka[2 i + h]), HD 64 k = k0 of all
+// four (ka[h]).  pf_read_v: the V^T operands of dimension tiles n0 .. n0 + 3
+// for one 32-key chunk (two transposing reads each, 16 rows apart).
+template <int HD>
+RFP4_DEV void pf_read_k(f16x8 (&ka)[4], uint32_t addr, uint32_t k0)
+{
+    if constexpr (HD == 128)
+        asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:4096\n\t"
+                     "ds_read_b128 %2, %5\n\tds_read_b128 %3, %5 offset:4096\n\ts_waitcnt lgkmcnt(0)"
+                     : "=&v"(ka[0]), "=&v"(ka[1]), "=&v"(ka[2]), "=&v"(ka[3])
+                     : "v"(addr ^ (k0 << 6)), "v"(addr ^ ((k0 + 1u) << 6)));
+    else
+        asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:2048\n\t"
+                     "ds_read_b128 %2, %4 offset:4096\n\tds_read_b128 %3, %4 offset:6144\n\ts_waitcnt lgkmcnt(0)"
+                     : "=&v"(ka[0]), "=&v"(ka[1]), "=&v"(ka[2]), "=&v"(ka[3])
+                     : "v"(addr ^ (k0 << 6)));
+}
+template <uint32_t RB>
+RFP4_DEV void pf_read_v(f16x8 (&va)[4], uint32_t addr, uint32_t n0)
+{
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    u32x2 lo[4], hi[4];
+    asm volatile("ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %1, %8 offset:%12\n\t"
+                 "ds_read_b64_tr_b16 %2, %9\n\tds_read_b64_tr_b16 %3, %9 offset:%12\n\t"
+                 "ds_read_b64_tr_b16 %4, %10\n\tds_read_b64_tr_b16 %5, %10 offset:%12\n\t"
+                 "ds_read_b64_tr_b16 %6, %11\n\tds_read_b64_tr_b16 %7, %11 offset:%12\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(lo[0]), "=&v"(hi[0]), "=&v"(lo[1]), "=&v"(hi[1]), "=&v"(lo[2]), "=&v"(hi[2]), "=&v"(lo[3]),
+                   "=&v"(hi[3])
+                 : "v"(addr ^ (n0 << 5)), "v"(addr ^ ((n0 + 1u) << 5)), "v"(addr ^ ((n0 + 2u) << 5)),
+                   "v"(addr ^ ((n0 + 3u) << 5)), "n"(16u * RB));
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+        va[i] = __builtin_bit_cast(f16x8, (u32x4v){lo[i].x, lo[i].y, hi[i].x, hi[i].y});
+    }
+}
 
 // One query tile: prompt rows r0 .. r0 + BQ of KV head blockIdx.y.  QO: the
 // kernel variant that can quantize its output rows (AttnPrefillArgs::q_codes;
@@ -48,7 +120,7 @@
 // (m the maximum, l and O rescaled by 2^(m_g - m) and summed): the serial
 // chain of blocks of a tile is KSP times shorter.
 template <int HD, int GT, int NW, bool QO, int KSP = 1>
-RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0)
+RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0, bool first)
 {
     const uint32_t pos0 = a.pos0, nrows = a.rows;
     constexpr int BQ = attn_prefill_rows(GT, NW);    // prompt rows per workgroup
@@ -59,21 +131,25 @@ RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0)
     // keys per block: 64 for head dim 64, 32 for 128 (measured: 8B 2048-row
     // kernel 96.4 us with 32, 103.2 with 64; TinyLlama 41.2 -> 37.8 us)
     constexpr int PF_BK = HD == 64 ? 64 : 32;
-    constexpr int KROW = HD + PF_KPAD, TROW = PF_BK + PF_TPAD;
-    constexpr int LPK = HD / 8;                      // 16-byte pieces per K/V row
-    constexpr int T = 64 * NW * KSP;                 // threads
-    constexpr int NP = KSP * PF_BK * LPK;            // 16-byte K (and V) pieces per staging step
-    constexpr int LD = (NP + T - 1) / T;             // K (and V) pieces per thread per step
-    constexpr bool LFULL = NP % T == 0;              // every thread loads LD pieces
+    constexpr uint32_t RB = 2u * HD;                 // bytes per K/V row
+    constexpr uint32_t LPR = HD / 8;                 // 16-byte chunks per row
+    constexpr int NWV = NW * KSP;                    // waves
+    constexpr uint32_t PB = PF_BK * RB / 1024u;      // 1 KB pieces of a block's K (and V)
+    constexpr uint32_t BLOCK = 2u * PF_BK * RB, STAGE = KSP * BLOCK;
+    constexpr int NI = (int)(STAGE / 1024u) / NWV;   // DMA instructions per wave and step
+    // stages: two steps of DMA lookahead with one block per step; two blocks per step leave the LDS for
+    // two workgroups per CU with one
+    constexpr uint32_t NST = KSP == 1 || NW == 8 ? 3 : 2;
     static_assert(NT % NW == 0 && MT >= 1, "tiles per wave");
-    static_assert(LFULL || LD == 1, "block load split");
-    __shared__ __align__(16) _Float16 ks[KSP][PF_BK][KROW];
-    __shared__ __align__(16) _Float16 vt[KSP][HD][TROW];
+    static_assert(NI * NWV * 1024 == (int)STAGE, "every wave copies the same number of pieces");
+    __shared__ __attribute__((aligned(1024))) uint8_t lds_raw[NST * STAGE];
+    pf_lds_u8 *lds = (pf_lds_u8 *)lds_raw;
 
-    const uint32_t kvh = blockIdx.y;
+    const uint32_t kvh = blockIdx.x % a.n_kv_heads;
     const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     // key group; wave within it (KSP = 1: the plain kernel's code, group 0)
-    const int kgrp = KSP > 1 ? (tid >> 6) / NW : 0, wave = KSP > 1 ? (tid >> 6) % NW : tid >> 6;
+    const int kgrp = KSP > 1 ? wid / NW : 0, wave = KSP > 1 ? wid % NW : wid;
     const uint32_t l16 = (uint32_t)lane & 15u, q4 = (uint32_t)lane >> 4;
     const uint32_t G = a.n_heads / a.n_kv_heads;
     const uint16_t *kc = a.kc + (size_t)kvh * a.hs;
@@ -116,65 +192,58 @@ RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0)
         for (int n = 0; n < NN; n++) o[mt][n] = {0.0f, 0.0f, 0.0f, 0.0f};
     }
 
-    // ---- K / V block loads: K piece (key tid / LPK, dims 8 (tid % LPK)), V
-    // piece (key tid % PF_BK, dims 8 (tid / PF_BK)) -- consecutive lanes take
-    // consecutive keys, so the transposed V writes fall on consecutive halves.
-    // Cached loads (each key row is read by every query tile of its KV head),
-    // two register sets: block b + 2's loads are issued when block b's data
-    // has gone to LDS, so each load has two blocks' compute to land.
-    // (each set one 8-word vector value per operand, piece j in words 4j ..
-    // 4j + 3: vectors stay in registers where the two sets' code is merged)
-    static_assert(LD == 1 || LD == 2 || LD == 4, "16-byte pieces per thread and block");
-    typedef uint32_t pf_vec __attribute__((ext_vector_type(4 * LD)));
-    pf_vec kr0, vr0, kr1, vr1;
-    // staging step I holds blocks I KSP .. I KSP + KSP - 1: piece p is piece
-    // p % (PF_BK LPK) of block slot p / (PF_BK LPK)
-#define RFP4_PF_LOAD(I, KR, VR)                                                                           \
-    do {                                                                                                  \
-        _Pragma("unroll") for (int j = 0; j < LD; j++) {                                                  \
-            /* threads past the step's pieces load the last one again (unused) */                         \
-            const uint32_t pa = min((uint32_t)tid + (uint32_t)T * (uint32_t)j, (uint32_t)NP - 1u);        \
-            const uint32_t kb0 = ((I) * KSP + pa / (PF_BK * LPK)) * PF_BK, p = pa % (PF_BK * LPK);       \
-            const uint32_t kk = min(kb0 + p / LPK, nk - 1u), kd = 8u * (p % LPK);                         \
-            const uint32_t vk = min(kb0 + p % PF_BK, nk - 1u), vd = 8u * (p / PF_BK);                      \
-            const u32x4 kx = *(const u32x4 *)(kc + (size_t)kk * a.ts + kd);                               \
-            const u32x4 vx = *(const u32x4 *)(vc + (size_t)vk * a.ts + vd);                               \
-            _Pragma("unroll") for (int i = 0; i < 4; i++) {                                               \
-                KR[4 * j + i] = kx[i];                                                                    \
-                VR[4 * j + i] = vx[i];                                                                    \
-            }                                                                                             \
-        }                                                                                                 \
-    } while (0)
-    // block b's K rows and transposed V rows into LDS, then block b + 2's loads into the same registers
-#define RFP4_PF_STAGE(I, KR, VR)                                                                          \
-    do {                                                                                                  \
-        __syncthreads(); /* the previous step's LDS reads are done */                                     \
-        _Pragma("unroll") for (int j = 0; j < LD; j++) {                                                  \
-            const uint32_t pa = (uint32_t)tid + (uint32_t)T * (uint32_t)j;                                \
-            if (!LFULL && pa >= (uint32_t)NP) break;                                                      \
-            const uint32_t sl = pa / (PF_BK * LPK), p = pa % (PF_BK * LPK);                              \
-            const u32x4 kx = {KR[4 * j], KR[4 * j + 1], KR[4 * j + 2], KR[4 * j + 3]};                    \
-            const u32x4 vx = {VR[4 * j], VR[4 * j + 1], VR[4 * j + 2], VR[4 * j + 3]};                    \
-            *(u32x4 *)&ks[sl][p / LPK][8u * (p % LPK)] = kx;                                              \
-            const uint32_t vk = p % PF_BK, vd = 8u * (p / PF_BK);                                          \
-            _Pragma("unroll") for (int i = 0; i < 4; i++) {                                               \
-                vt[sl][vd + 2u * i][vk] = __builtin_bit_cast(_Float16, (uint16_t)(vx[i] & 0xFFFFu));      \
-                vt[sl][vd + 2u * i + 1u][vk] = __builtin_bit_cast(_Float16, (uint16_t)(vx[i] >> 16));     \
-            }                                                                                             \
-        }                                                                                                 \
-        __syncthreads();                                                                                  \
-        RFP4_PF_LOAD((I) + 2u, KR, VR);                                                                   \
-    } while (0)
-    // Every load is issued on every path (keys clamped to the last one, so a
-    // block past the end re-reads it): the compiler's wait for a set then
-    // counts exactly the other set's loads behind it, where paths with and
-    // without a load would make it wait for both sets.
-    RFP4_PF_LOAD(0u, kr0, vr0);
-    RFP4_PF_LOAD(1u, kr1, vr1);
+    // ---- K / V staging: DMA (global_load_lds), no registers.  A step's stage
+    // holds KSP blocks, each PF_BK K rows then PF_BK V rows of HD halves, row
+    // major, the 16-byte chunks of a row XOR-swizzled (pf_kswz, pf_vswz).  One
+    // DMA instruction fills 1 KB (64 / LPR rows of LPR chunks): lane l's chunk
+    // goes to physical chunk l % LPR, so it fetches logical chunk l % LPR ^
+    // swizzle(row).  Keys past the last one re-read it (finite values, masked
+    // scores), so every wave issues the same DMAs in every step.
+    // Steps inside the context use 32-bit lane offsets from a uniform base (one
+    // scalar add per step instead of a 64-bit address per lane and copy); the
+    // last ones, and strides past 4 GB, clamp each row.
+    constexpr uint32_t RPI = 64u / LPR; // rows per DMA instruction
+    static_assert((NWV * RPI) % 16u == 0u && (NWV % PB == 0u || PB % NWV == 0u), "the same swizzle for every copy of a lane");
+    const uint32_t row0 = ((uint32_t)wid % PB) * RPI + (uint32_t)lane / LPR, ch = (uint32_t)lane % LPR;
+    const uint32_t lck = ch ^ pf_kswz<HD>(row0), lcv = ch ^ pf_vswz<HD>(row0);
+    const uint32_t voffk = 2u * (row0 * (uint32_t)a.ts + 8u * lck), voffv = 2u * (row0 * (uint32_t)a.ts + 8u * lcv);
+    const bool small = a.ts < (1ull << 24); // PF_BK rows of ts halves stay under 4 GB
+    auto stage_dma = [&](uint32_t step, uint32_t buf) {
+        const bool whole = small && (step + 1u) * (KSP * PF_BK) <= nk;
+#pragma unroll
+        for (int j = 0; j < NI; j++) {
+            const uint32_t c = (uint32_t)wid + (uint32_t)(NWV * j); // 1 KB piece of the stage
+            const uint32_t slot = c / (2u * PB), isv = (c / PB) & 1u;
+            const uint32_t k0 = (step * KSP + slot) * PF_BK + ((uint32_t)(NWV * j) % PB) * RPI; // row0's first key
+            const uint16_t *base = isv ? vc : kc;
+            pf_lds_u8 *dst = lds + buf * STAGE + 1024u * c;
+            if (whole) {
+                const uint8_t *src = (const uint8_t *)(base + (size_t)k0 * a.ts);
+                __builtin_amdgcn_global_load_lds((pf_glb_void *)(src + (isv ? voffv : voffk)), dst, 16, 0, 0);
+            } else {
+                const uint16_t *src = base + (size_t)min(k0 + row0, nk - 1u) * a.ts + 8u * (isv ? lcv : lck);
+                __builtin_amdgcn_global_load_lds((pf_glb_void *)src, dst, 16, 0, 0);
+            }
+        }
+    };
+    // this lane's LDS byte addresses inside a stage.  K: row l16 of the first
+    // 16 keys, chunk q4; key quarter h and dimension step k are 16 rows and an
+    // XOR of 4 k chunks away.  V: the transposing read (ds_read_b64_tr_b16:
+    // lane j of 16 gives the address of 4 halves, row j / 4 of a 4 x 16 block,
+    // columns 4 (j % 4) .. +3, and receives column j of its 4 rows) of keys
+    // 4 q4 .. +3 and dimensions 0 .. 15; dimension tile n is an XOR of 2 n
+    // chunks away, the chunk's other 16 keys 16 rows.
+    const uint32_t lds0 = (uint32_t)(uintptr_t)lds + (uint32_t)kgrp * BLOCK;
+    const uint32_t kaddr = lds0 + l16 * RB + ((q4 ^ pf_kswz<HD>(l16)) << 4);
+    const uint32_t vrow = 4u * q4 + (l16 >> 2);
+    const uint32_t vaddr = lds0 + PF_BK * RB + vrow * RB + ((((l16 & 3u) >> 1) ^ pf_vswz<HD>(vrow)) << 4) + 8u * (l16 & 1u);
+    if (!first) __syncthreads(); // the previous tile's LDS reads are done
+#pragma unroll
+    for (uint32_t i = 0; i + 1u < NST; i++) stage_dma(i, i);
 
-    // the block's scores, softmax and P V from the staged K / V (this key
+    // the block's scores, softmax and P V from the stage at byte sb (this key
     // group's block b of the step in slot kgrp; none past the last block)
-    auto block = [&](uint32_t b) {
+    auto block = [&](uint32_t b, uint32_t sb) {
         if (KSP > 1 && b >= nblk) return; // the same for the whole key group
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
@@ -182,55 +251,67 @@ RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0)
             // ---- S^T = K Q^T for the block's 16-key quarters h: accumulator r
             // of lane l is key 16 h + 4 q4 + r of row l16
             constexpr int NQ = PF_BK / 16;
+            static_assert(NQ * KS == 8 && 4 % NQ == 0, "pf_read_k");
             f32x4 s[NQ];
 #pragma unroll
-            for (int h = 0; h < NQ; h++) {
-                s[h] = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int h = 0; h < NQ; h++) s[h] = {0.0f, 0.0f, 0.0f, 0.0f};
+            constexpr int KB = 4 / NQ; // dimension steps per read
 #pragma unroll
-                for (int k = 0; k < KS; k++) {
-                    const f16x8 ka = *(const f16x8 *)&ks[kgrp][16u * h + l16][32 * k + 8u * q4];
-                    s[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qa[mt][k], s[h], 0, 0, 0);
-                    s[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql[mt][k], s[h], 0, 0, 0);
+            for (int k0 = 0; k0 < KS; k0 += KB) {
+                f16x8 ka[4];
+                pf_read_k<HD>(ka, kaddr + sb, (uint32_t)k0);
+#pragma unroll
+                for (int i = 0; i < KB; i++) {
+#pragma unroll
+                    for (int h = 0; h < NQ; h++)
+                        s[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[i * NQ + h], qa[mt][k0 + i], s[h], 0, 0, 0);
+#pragma unroll
+                    for (int h = 0; h < NQ; h++)
+                        s[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[i * NQ + h], ql[mt][k0 + i], s[h], 0, 0, 0);
                 }
             }
-            // ---- causal mask (only in blocks that reach past the tile's first
-            // row), online softmax (base 2) of the lane's row
-            const uint32_t row0 = r0 + 16u * (t / GT);
-            const uint32_t qpos = pos0 + min(row0 + l16, nrows - 1u);
-            const bool masked = (b + 1u) * PF_BK > pos0 + min(row0, nrows - 1u) + 1u; // the same for the whole wave
+            // ---- causal mask (only in blocks that reach past the tile's first row)
+            const uint32_t row0t = r0 + 16u * (t / GT);
+            const bool masked = (b + 1u) * PF_BK > pos0 + min(row0t, nrows - 1u) + 1u; // the same for the whole wave
             float p[4 * NQ];
+#pragma unroll
+            for (int h = 0; h < NQ; h++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) p[4 * h + r] = s[h][r];
             if (masked) {
+                const uint32_t qpos = pos0 + min(row0t + l16, nrows - 1u);
 #pragma unroll
                 for (int h = 0; h < NQ; h++)
 #pragma unroll
                     for (int r = 0; r < 4; r++) {
                         const uint32_t key = b * PF_BK + 16u * h + 4u * q4 + (uint32_t)r;
-                        p[4 * h + r] = key <= qpos ? s[h][r] : -3.402823466e38f;
+                        if (key > qpos) p[4 * h + r] = -3.402823466e38f;
                     }
-            } else {
-#pragma unroll
-                for (int h = 0; h < NQ; h++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) p[4 * h + r] = s[h][r];
             }
-            // the maximum of the raw scores, then scaled: rounding is monotonic,
-            // so this is the maximum of the scaled scores
+            // ---- online softmax (base 2) of the lane's row.  The subtracted
+            // maximum is raised only when a score of the row exceeds it by
+            // more than 8 (p is at most 2^8 and keeps its relative precision
+            // in hi + lo; l and O are f32): in the common block there is no
+            // cross-lane step and no O rescale (32 of 150 VALU instructions),
+            // and the sum stays per lane until the end.
             float mx = p[0];
 #pragma unroll
             for (int i = 1; i < 4 * NQ; i++) mx = fmaxf(mx, p[i]);
-            mx = xor32_max(xor16_max(mx)) * scale;
-            const float mnew = fmaxf(mrun[mt], mx);
-            const float alpha = __builtin_amdgcn_exp2f(mrun[mt] - mnew);
-            mrun[mt] = mnew;
-            float ls = 0.0f;
+            mx *= scale; // rounding is monotonic: the maximum of the scaled scores
+            if (__any(mx > mrun[mt] + 8.0f)) {
+                const float rowmax = xor32_max(xor16_max(mx));
+                const float mnew = rowmax > mrun[mt] + 8.0f ? rowmax : mrun[mt]; // a row's own choice, whatever its wave holds
+                const float alpha = __builtin_amdgcn_exp2f(mrun[mt] - mnew);
+                mrun[mt] = mnew;
+                lrun[mt] *= alpha;
+#pragma unroll
+                for (int n = 0; n < NN; n++) o[mt][n] *= alpha;
+            }
 #pragma unroll
             for (int i = 0; i < 4 * NQ; i++) {
-                p[i] = __builtin_amdgcn_exp2f(p[i] * scale - mnew);
-                ls += p[i];
+                p[i] = __builtin_amdgcn_exp2f(fmaf(p[i], scale, -mrun[mt]));
+                lrun[mt] += p[i];
             }
-            lrun[mt] = fmaf(lrun[mt], alpha, xor32_sum(xor16_sum(ls)));
-#pragma unroll
-            for (int n = 0; n < NN; n++) o[mt][n] *= alpha;
             // ---- O^T += V^T P^T per 32-key chunk c (quarters 2c, 2c + 1): P^T as
             // hi + lo operands straight from the registers; V^T dimension row
             // 16 n + l16 at the lane's 8 keys of the chunk
@@ -239,35 +320,49 @@ RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0)
                 f16x8 pb, pl;
                 split_hi_lo8_mix(p + 8 * c, pb, pl);
 #pragma unroll
-                for (int n = 0; n < NN; n++) {
-                    const _Float16 *vrow = &vt[kgrp][16u * n + l16][32u * c + 4u * q4];
-                    typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-                    const f16x4 v0 = *(const f16x4 *)vrow, v1 = *(const f16x4 *)(vrow + 16);
-                    const f16x8 va = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-                    o[mt][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pb, o[mt][n], 0, 0, 0);
-                    o[mt][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl, o[mt][n], 0, 0, 0);
+                for (int n0 = 0; n0 < NN; n0 += 4) {
+                    f16x8 va[4];
+                    pf_read_v<RB>(va, vaddr + sb + (uint32_t)c * 32u * RB, (uint32_t)n0);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        o[mt][n0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[i], pb, o[mt][n0 + i], 0, 0, 0);
+                        o[mt][n0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[i], pl, o[mt][n0 + i], 0, 0, 0);
+                    }
                 }
             }
         }
     };
-    uint32_t it = 0;
-    for (; it + 1u < niter; it += 2u) {
-        RFP4_PF_STAGE(it, kr0, vr0);
-        block(it * KSP + (uint32_t)kgrp);
-        RFP4_PF_STAGE(it + 1u, kr1, vr1);
-        block((it + 1u) * KSP + (uint32_t)kgrp);
+    // Step i: wait for this wave's DMAs of step i (those of the NST - 2 steps
+    // behind it may be in flight), then the barrier: every wave's copies of
+    // step i are in LDS and every wave is past its reads of step i - 1, whose
+    // buffer the DMAs of step i + NST - 1 then overwrite.
+    uint32_t buf = 0;
+    for (uint32_t it = 0; it < niter; it++) {
+        __builtin_amdgcn_s_waitcnt(PF_VMCNT(NI * (NST - 2u)));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        stage_dma(it + NST - 1u, buf == 0u ? NST - 1u : buf - 1u);
+        block(it * KSP + (uint32_t)kgrp, buf * STAGE);
+        buf = buf + 1u == NST ? 0u : buf + 1u;
     }
-    if (it < niter) {
-        RFP4_PF_STAGE(it, kr0, vr0);
-        block(it * KSP + (uint32_t)kgrp);
-    }
-#undef RFP4_PF_STAGE
-#undef RFP4_PF_LOAD
+    // the last DMAs (past the end) land before the LDS is used again
+    __builtin_amdgcn_s_waitcnt(PF_VMCNT(0));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+
+    // the row's sum over its four lanes
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) lrun[mt] = xor32_sum(xor16_sum(lrun[mt]));
 
     if constexpr (KSP > 1) {
         // ---- the key groups' states merged into group 0's: groups 1.. put
         // (O, m, l) in LDS (lane-contiguous words), group 0 combines
-        __shared__ float mg[KSP - 1][NW][MT][NN * 4 + 2][64];
+        // (in the stages, free after the loop)
+        typedef float pf_mg[NW][MT][NN * 4 + 2][64];
+        static_assert(sizeof(pf_mg) * (KSP - 1) <= NST * STAGE, "the merged states in the stages");
+        pf_mg *mg = (pf_mg *)lds_raw;
         if (kgrp > 0) {
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) {
@@ -357,16 +452,20 @@ RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0)
     }
 }
 
-// Workgroup x of KV head blockIdx.y: query tile x, or, paired, tiles
-// ntiles - 1 - x (the longer causal range, first) and x, so that every
-// workgroup walks ntiles + 1 key ranges' worth of blocks.
+// Grid (one dimension, n_kv_heads x tiles): consecutive workgroups take the same query tile
+// of every KV head, the longest causal range first, so that the short
+// ones fill the end of the launch; with 8 KV heads each XCD (workgroup id % 8)
+// keeps one head's K/V in its L2.
+// Workgroup y of a head: query tile ntiles - 1 - y, or, paired, tiles ntiles
+// - 1 - y and y, so that every workgroup walks ntiles + 1 key ranges' worth of
+// blocks.
 template <int HD, int GT, int NW = 4, bool QO = false, int KSP = 1>
 RFP4_DEV void attn_prefill_body(const AttnPrefillArgs &a)
 {
     constexpr uint32_t BQ = (uint32_t)attn_prefill_rows(GT, NW);
-    const uint32_t ntiles = (a.rows + BQ - 1u) / BQ, x = blockIdx.x;
-    const uint32_t t0 = a.paired ? ntiles - 1u - x : x;
-    const uint32_t npass = a.paired && x < t0 ? 2u : 1u;
+    const uint32_t ntiles = (a.rows + BQ - 1u) / BQ, y = blockIdx.x / a.n_kv_heads, t0 = ntiles - 1u - y;
+    const uint32_t npass = a.paired && y < t0 ? 2u : 1u;
 #pragma nounroll
-    for (uint32_t pass = 0; pass < npass; pass++) attn_prefill_tile<HD, GT, NW, QO, KSP>(a, (pass == 0 ? t0 : x) * BQ);
+    for (uint32_t pass = 0; pass < npass; pass++)
+        attn_prefill_tile<HD, GT, NW, QO, KSP>(a, (pass == 0 ? t0 : y) * BQ, pass == 0);
 }

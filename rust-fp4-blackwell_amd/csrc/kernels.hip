@@ -106,16 +106,16 @@ ATTN_KERNELS(128, f32, float)
 ATTN_KERNELS(128, f16, uint16_t)
 // rfp4_attn_prefill_hd<HD>_g<group>_w<waves per workgroup>[_q: the output
 // rows quantized to MXFP4 as well, AttnPrefillArgs::q_codes]
-#define K512Q extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+#define K512Q extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 #define ATTN_PREFILL_KERNELS(HD) \
     K256 void rfp4_attn_prefill_hd##HD##_g1_w4(AttnPrefillArgs a) { attn_prefill_body<HD, 1, 4>(a); } \
     K256 void rfp4_attn_prefill_hd##HD##_g2_w4(AttnPrefillArgs a) { attn_prefill_body<HD, 2, 4>(a); } \
     K256 void rfp4_attn_prefill_hd##HD##_g4_w4(AttnPrefillArgs a) { attn_prefill_body<HD, 4, 4>(a); } \
     K256 void rfp4_attn_prefill_hd##HD##_g8_w4(AttnPrefillArgs a) { attn_prefill_body<HD, 8, 4>(a); } \
-    K512 void rfp4_attn_prefill_hd##HD##_g1_w8(AttnPrefillArgs a) { attn_prefill_body<HD, 1, 8>(a); } \
-    K512 void rfp4_attn_prefill_hd##HD##_g2_w8(AttnPrefillArgs a) { attn_prefill_body<HD, 2, 8>(a); } \
-    K512 void rfp4_attn_prefill_hd##HD##_g4_w8(AttnPrefillArgs a) { attn_prefill_body<HD, 4, 8>(a); } \
-    K512 void rfp4_attn_prefill_hd##HD##_g8_w8(AttnPrefillArgs a) { attn_prefill_body<HD, 8, 8>(a); } \
+    K512Q void rfp4_attn_prefill_hd##HD##_g1_w8(AttnPrefillArgs a) { attn_prefill_body<HD, 1, 8>(a); } \
+    K512Q void rfp4_attn_prefill_hd##HD##_g2_w8(AttnPrefillArgs a) { attn_prefill_body<HD, 2, 8>(a); } \
+    K512Q void rfp4_attn_prefill_hd##HD##_g4_w8(AttnPrefillArgs a) { attn_prefill_body<HD, 4, 8>(a); } \
+    K512Q void rfp4_attn_prefill_hd##HD##_g8_w8(AttnPrefillArgs a) { attn_prefill_body<HD, 8, 8>(a); } \
     K256 void rfp4_attn_prefill_hd##HD##_g1_w4_q(AttnPrefillArgs a) { attn_prefill_body<HD, 1, 4, true>(a); } \
     K256 void rfp4_attn_prefill_hd##HD##_g2_w4_q(AttnPrefillArgs a) { attn_prefill_body<HD, 2, 4, true>(a); } \
     K256 void rfp4_attn_prefill_hd##HD##_g4_w4_q(AttnPrefillArgs a) { attn_prefill_body<HD, 4, 4, true>(a); } \
@@ -129,14 +129,28 @@ ATTN_PREFILL_KERNELS(128)
 // key-split variants (two key groups of 4 waves each, _s2; groups of up to 4
 // query heads: runtime.cpp attn_prefill_launch)
 #define ATTN_PREFILL_SPLIT_KERNELS(HD) \
-    K512 void rfp4_attn_prefill_hd##HD##_g1_w4_s2(AttnPrefillArgs a) { attn_prefill_body<HD, 1, 4, false, 2>(a); } \
-    K512 void rfp4_attn_prefill_hd##HD##_g2_w4_s2(AttnPrefillArgs a) { attn_prefill_body<HD, 2, 4, false, 2>(a); } \
-    K512 void rfp4_attn_prefill_hd##HD##_g4_w4_s2(AttnPrefillArgs a) { attn_prefill_body<HD, 4, 4, false, 2>(a); } \
+    K512Q void rfp4_attn_prefill_hd##HD##_g1_w4_s2(AttnPrefillArgs a) { attn_prefill_body<HD, 1, 4, false, 2>(a); } \
+    K512Q void rfp4_attn_prefill_hd##HD##_g2_w4_s2(AttnPrefillArgs a) { attn_prefill_body<HD, 2, 4, false, 2>(a); } \
+    K512Q void rfp4_attn_prefill_hd##HD##_g4_w4_s2(AttnPrefillArgs a) { attn_prefill_body<HD, 4, 4, false, 2>(a); } \
     K512Q void rfp4_attn_prefill_hd##HD##_g1_w4_q_s2(AttnPrefillArgs a) { attn_prefill_body<HD, 1, 4, true, 2>(a); } \
     K512Q void rfp4_attn_prefill_hd##HD##_g2_w4_q_s2(AttnPrefillArgs a) { attn_prefill_body<HD, 2, 4, true, 2>(a); } \
     K512Q void rfp4_attn_prefill_hd##HD##_g4_w4_q_s2(AttnPrefillArgs a) { attn_prefill_body<HD, 4, 4, true, 2>(a); }
 ATTN_PREFILL_SPLIT_KERNELS(64)
 ATTN_PREFILL_SPLIT_KERNELS(128)
+// 16 waves: four key groups of 4 waves (_s4, groups of up to 4 heads), two of
+// 8 (groups of 8)
+#define ATTN_PREFILL_SPLIT16_KERNELS(HD) \
+    K1024 void rfp4_attn_prefill_hd##HD##_g1_w4_s4(AttnPrefillArgs a) { attn_prefill_body<HD, 1, 4, false, 4>(a); } \
+    K1024 void rfp4_attn_prefill_hd##HD##_g2_w4_s4(AttnPrefillArgs a) { attn_prefill_body<HD, 2, 4, false, 4>(a); } \
+    K1024 void rfp4_attn_prefill_hd##HD##_g4_w4_s4(AttnPrefillArgs a) { attn_prefill_body<HD, 4, 4, false, 4>(a); } \
+    K1024 void rfp4_attn_prefill_hd##HD##_g8_w8_s2(AttnPrefillArgs a) { attn_prefill_body<HD, 8, 8, false, 2>(a); } \
+    K1024 void rfp4_attn_prefill_hd##HD##_g1_w4_q_s4(AttnPrefillArgs a) { attn_prefill_body<HD, 1, 4, true, 4>(a); } \
+    K1024 void rfp4_attn_prefill_hd##HD##_g2_w4_q_s4(AttnPrefillArgs a) { attn_prefill_body<HD, 2, 4, true, 4>(a); } \
+    K1024 void rfp4_attn_prefill_hd##HD##_g4_w4_q_s4(AttnPrefillArgs a) { attn_prefill_body<HD, 4, 4, true, 4>(a); } \
+    K1024 void rfp4_attn_prefill_hd##HD##_g8_w8_q_s2(AttnPrefillArgs a) { attn_prefill_body<HD, 8, 8, true, 2>(a); }
+ATTN_PREFILL_SPLIT16_KERNELS(64)
+ATTN_PREFILL_SPLIT16_KERNELS(128)
+#undef ATTN_PREFILL_SPLIT16_KERNELS
 #undef ATTN_PREFILL_SPLIT_KERNELS
 // ---- fused q|k|v GEMV + attention: rfp4_qkva_hd<HD>_g<group>[_t: tagged merge]
 // (device/qkva.h).  HD 64 with K = 2048 (one slice, R = 2 or 1 (_r1), the

@@ -624,8 +624,8 @@ extern "C" int rfp4_debug_prefill_waves(int waves)
 extern "C" int rfp4_debug_prefill_ksplit(int groups)
 {
     using namespace rfp4;
-    if (groups < 0 || groups > 2)
-        return set_error(RFP4_E_INVALID, "prefill attention key groups must be 0 (auto), 1 (one) or 2 (two where compiled)");
+    if (groups < 0 || groups > 4 || groups == 3)
+        return set_error(RFP4_E_INVALID, "prefill attention key groups must be 0 (auto), 1 (one), or 2 or 4 where compiled");
     t_prefill_ksplit = groups;
     return RFP4_OK;
 }
@@ -756,39 +756,44 @@ int attn_prefill_launch(const AttnPrefillArgs &a, uint32_t head_dim, hipStream_t
                          a.n_kv_heads);
     if (a.rows == 0) return RFP4_OK;
     const uint32_t g = attn_group_pad(a.n_heads / a.n_kv_heads);
-    // 8 waves per workgroup (one 16-row tile each, twice the rows per staged
-    // K/V block, 118 VGPRs) wherever that still gives every CU a workgroup
-    // or the tile height does not change (8 query heads per KV head); else 4.
-    // Measured: 8B prefill 2048 tokens 23.5 -> 22.3 ms, 512 tokens 8.52 ->
-    // 8.76 ms (128 workgroups); TinyLlama 512 / 2048 tokens 3.02 -> 2.83 /
-    // 7.69 -> 7.15 ms.
-    uint32_t waves = 4u;
-    {
-        const uint32_t b8 = (uint32_t)attn_prefill_rows((int)g, 8), b4 = (uint32_t)attn_prefill_rows((int)g, 4);
-        const uint64_t grid8 = (uint64_t)((a.rows + b8 - 1) / b8) * a.n_kv_heads;
-        if (b8 == b4 || (g_rt && grid8 >= (uint64_t)g_rt->num_cus)) waves = 8u;
-    }
+    // 4 waves (16 prompt rows of 4 heads, one 16-row tile per wave) per key
+    // group, 8 where the KV head has 8 query heads.
+    uint32_t waves = g == 8u ? 8u : 4u;
     if (t_prefill_waves) waves = (uint32_t)t_prefill_waves;
     const uint32_t bq = (uint32_t)attn_prefill_rows((int)g, (int)waves); // prompt rows per workgroup
     const uint32_t ntiles = (a.rows + bq - 1) / bq;
-    // Causal tiles differ in length (tile t walks t + 1 key ranges' worth of
-    // blocks); pairing tile t with ntiles - 1 - t in one workgroup evens them
-    // out wherever the halved grid still gives every CU a workgroup.
-    bool paired = ntiles >= 2 && g_rt && (uint64_t)((ntiles + 1) / 2) * a.n_kv_heads >= (uint64_t)g_rt->num_cus;
-    if (t_prefill_pairing) paired = t_prefill_pairing == 2;
+    const uint64_t keys = (uint64_t)a.pos0 + a.rows, wgs = (uint64_t)ntiles * a.n_kv_heads;
+    // Key groups per workgroup (alternate key blocks, the states merged at the
+    // end): a tile's serial chain of blocks halves or quarters, for a merge of
+    // 1-3 us.  Measured (us, 1 / 2 / 4 groups of 4 waves): Llama-3-8B heads, 64
+    // rows 7.1 / 7.3 / 9.9, 512 rows 19.6 / 15.3 / 16.8, 2048 rows 83.7 / 76.6 /
+    // 91.9, 100 rows after 4000 keys 108 / 63.5 / 56.1; 8 heads of one group
+    // each, 1024 rows 31.9 / 22.0 / 21.8, 2048 rows 59.7 / 38.9 / 35.7.  Two
+    // groups of 8 waves (8 query heads per KV head; 1 / 2 groups): TinyLlama
+    // heads, 333 rows 10.6 / 11.2, 700 rows 17.0 / 16.9, 2048 rows 49.6 / 44.1;
+    // 100 rows after 4000 keys 69.2 / 59.5.  So: four groups for long chains
+    // where a workgroup per CU holds the grid (16 waves fill a CU), else two,
+    // and one for contexts of a few blocks.
+    const uint64_t cus = g_rt ? (uint64_t)g_rt->num_cus : 256u;
+    uint32_t ks = waves == 8u ? (g == 8u && keys > 512u ? 2u : 1u) : g == 8u || keys <= 64u ? 1u : keys > 1024u && wgs <= cus ? 4u : 2u;
+    if (t_prefill_ksplit) {
+        ks = (uint32_t)t_prefill_ksplit;
+        if (ks == 4u && !(waves == 4u && g < 8u)) ks = 2u;
+        if (ks == 2u && !((waves == 4u && g < 8u) || (waves == 8u && g == 8u))) ks = 1u;
+    }
+    // Pairing tile t with ntiles - 1 - t in one workgroup evens out the causal
+    // ranges of a grid of one workgroup per CU; no longer chosen (two
+    // workgroups per CU, the longest first, are as fast or faster: 2048 rows of
+    // 8B heads 76.6 against 82.6 us paired).
+    const bool paired = t_prefill_pairing == 2;
     char name[48];
-    // two key groups of 4 waves per workgroup (alternate key blocks, the
-    // states merged at the end: the serial chain of blocks halves) where the
-    // plan is 4 waves and groups of up to 4 heads.  Measured: 8B prefill 512
-    // tokens 5.29-5.35 -> 5.18-5.24 ms; TinyLlama (8 heads, 8 waves) slower
-    // split (2.21 -> 2.24 ms), so not compiled there.
-    const bool ksplit = t_prefill_ksplit != 1 && waves == 4u && g < 8u;
-    snprintf(name, sizeof name, "rfp4_attn_prefill_hd%u_g%u_w%u%s%s", head_dim, g, waves, a.q_codes ? "_q" : "",
-             ksplit ? "_s2" : "");
+    char sfx[8] = "";
+    if (ks > 1u) snprintf(sfx, sizeof sfx, "_s%u", ks);
+    snprintf(name, sizeof name, "rfp4_attn_prefill_hd%u_g%u_w%u%s%s", head_dim, g, waves, a.q_codes ? "_q" : "", sfx);
     AttnPrefillArgs args = a;
     args.paired = paired ? 1u : 0u;
     const uint32_t gx = paired ? (ntiles + 1) / 2 : ntiles;
-    return launch(name, dim3(gx, a.n_kv_heads), dim3(64u * waves * (ksplit ? 2u : 1u)), s, &args);
+    return launch(name, dim3(a.n_kv_heads * gx), dim3(64u * waves * ks), s, &args);
 }
 
 uint32_t attn_group_pad(uint32_t group) { return group <= 1u ? 1u : group <= 2u ? 2u : group <= 4u ? 4u : 8u; }
