@@ -482,13 +482,14 @@ static int enqueue_prefill(llama_engine *e, uint32_t n, uint32_t pos0)
         // where the plan has that kernel (bit-identical to the row kernel
         // after the GEMM; not when the stage test hook wants the GEMM's output)
         const uint64_t kv_hs = (uint64_t)e->max_seq_alloc * hd;
-        if (stop != (int)(10u * l + 1u) && prefill_rope_mode() == 0 && gemm_rope_ok(n, nqkv, c.dim, hd)) {
+        const bool rope_ok = gemm_rope_ok(n, nqkv, c.dim, hd);
+        if (stop != (int)(10u * l + 1u) && prefill_rope_mode() == 0 && rope_ok) {
             const GemmRope gr{e->cos_tab, e->sin_tab, kc, vc, hd, kv_hs, pos0, qd, kvd, hd};
             if ((rc = gemm_rope_launch(s, n, nqkv, c.dim, e->pf_codes, e->pf_scales, e->pf_scales_t, w.qkv_c, w.qkv_s,
                                        w.qkv_st, e->pf_c, gr))) return rc;
         } else {
             if ((rc = gemm_launch(s, n, nqkv, c.dim, e->pf_codes, e->pf_scales, e->pf_scales_t, w.qkv_c, w.qkv_s,
-                                  w.qkv_st, e->pf_c, e->gemm_part))) return rc;
+                                  w.qkv_st, e->pf_c, e->gemm_part, false, rope_ok ? GEMM_ROPE : GEMM_LAYER))) return rc;
             RFP4_PF_STAGE(1);
             RopeRowsArgs ra{};
             ra.qkv = e->pf_c; ra.cosv = e->cos_tab; ra.sinv = e->sin_tab; ra.kc = kc; ra.vc = vc;
@@ -534,7 +535,7 @@ static int enqueue_prefill(llama_engine *e, uint32_t n, uint32_t pos0)
         // arithmetic; not when the stage test hook wants the GEMM's output)
         const bool o_in_x = stop != (int)(10u * l + 5u) && gemm_accumulate_ok(n, c.dim, qd);
         if ((rc = gemm_launch(s, n, c.dim, qd, e->pf_codes, e->pf_scales, e->pf_scales_t, w.o_c, w.o_s, w.o_st,
-                              o_in_x ? e->pf_x : e->pf_c, e->gemm_part, o_in_x))) return rc;
+                              o_in_x ? e->pf_x : e->pf_c, e->gemm_part, o_in_x, GEMM_LAYER))) return rc;
         RFP4_PF_STAGE(5);
         na.w = e->norm_ffn + (size_t)l * c.dim;
         na.add = o_in_x ? nullptr : e->pf_c; // x += O projection (unless added already), then the FFN norm
@@ -542,15 +543,16 @@ static int enqueue_prefill(llama_engine *e, uint32_t n, uint32_t pos0)
         e->pf_q_alt = false;
         RFP4_PF_STAGE(6);
         // gate|up: SwiGLU and the MXFP4 rows of its output in the GEMM's
-        // epilogue where the plan is the 256x256 ping-pong tile (no f32
-        // gate|up output; not when the stage test hook wants that output)
-        if (stop != (int)(10u * l + 7u) && prefill_swiglu_mode() == 0 && gemm_swiglu_ok(n, c.ffn, c.dim)) {
+        // epilogue where that is estimated faster (no f32 gate|up output;
+        // not when the stage test hook wants that output)
+        const bool swiglu_ok = gemm_swiglu_ok(n, c.ffn, c.dim);
+        if (stop != (int)(10u * l + 7u) && prefill_swiglu_mode() == 0 && swiglu_ok) {
             if ((rc = gemm_swiglu_launch(s, n, c.ffn, c.dim, e->pf_codes, e->pf_scales, e->pf_scales_t, w.gu_c, w.gu_s,
                                          w.gu_st, e->pf_codes2, e->pf_scales2, e->pf_scales_t2))) return rc;
             e->pf_q_alt = true;
         } else {
             if ((rc = gemm_launch(s, n, 2 * c.ffn, c.dim, e->pf_codes, e->pf_scales, e->pf_scales_t, w.gu_c, w.gu_s,
-                                  w.gu_st, e->pf_c, e->gemm_part))) return rc;
+                                  w.gu_st, e->pf_c, e->gemm_part, false, swiglu_ok ? GEMM_SWIGLU : GEMM_LAYER))) return rc;
             RFP4_PF_STAGE(7);
             RowsArgs sa{};
             sa.x = e->pf_c; sa.codes = e->pf_codes; sa.scales = e->pf_scales; sa.scales_t = e->pf_scales_t;
@@ -565,7 +567,7 @@ static int enqueue_prefill(llama_engine *e, uint32_t n, uint32_t pos0)
         uint8_t *dst_ = e->pf_q_alt ? e->pf_scales_t2 : e->pf_scales_t;
         down_in_x = stop != (int)(10u * l + 9u) && gemm_accumulate_ok(n, c.dim, c.ffn);
         if ((rc = gemm_launch(s, n, c.dim, c.ffn, dc, ds, dst_, w.d_c, w.d_s, w.d_st, down_in_x ? e->pf_x : e->pf_c,
-                              e->gemm_part, down_in_x))) return rc;
+                              e->gemm_part, down_in_x, GEMM_LAYER))) return rc;
         RFP4_PF_STAGE(9);
         // x += down projection: in its GEMM, else by the next layer's first norm, after the last layer here
         if (l + 1 == c.n_layers && !down_in_x && (rc = residual(s, n * c.dim, e->pf_c, e->pf_x))) return rc;

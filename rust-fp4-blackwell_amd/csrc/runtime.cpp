@@ -1207,28 +1207,13 @@ namespace {
 struct GemmTile {
     uint32_t bm, bn;
     const char *name;
-    uint32_t occ; // workgroups per CU (registers / LDS of the compiled kernel)
 };
 // Compiled tile shapes (kernels.hip GEMM_KERNEL), largest first.
-// (occ: workgroups per CU of the double-buffered kernel as this build compiles
-// it, used when no runtime is initialised; gemm_occ asks the runtime)
 constexpr GemmTile kGemmTiles[] = {
-    {256, 256, "rfp4_gemm_256x256", 1}, {256, 128, "rfp4_gemm_256x128", 1}, {128, 128, "rfp4_gemm_128x128", 1},
-    {64, 128, "rfp4_gemm_64x128", 2},   {32, 128, "rfp4_gemm_32x128", 3},
+    {256, 256, "rfp4_gemm_256x256"}, {256, 128, "rfp4_gemm_256x128"}, {128, 128, "rfp4_gemm_128x128"},
+    {64, 128, "rfp4_gemm_64x128"},   {32, 128, "rfp4_gemm_32x128"},
 };
 constexpr int kGemmNumTiles = (int)(sizeof(kGemmTiles) / sizeof(kGemmTiles[0]));
-// Workgroups of tile i's double-buffered kernel that fit one CU (registers
-// and LDS of the compiled code object), asked once per process.
-uint32_t gemm_occ(int i)
-{
-    static std::atomic<uint32_t> occ[kGemmNumTiles];
-    uint32_t v = occ[i].load(std::memory_order_relaxed);
-    if (v) return v;
-    int per_cu = 0;
-    if (!g_rt || kernel_occupancy(kGemmTiles[i].name, 256, 0, &per_cu) || per_cu <= 0) return kGemmTiles[i].occ;
-    occ[i].store((uint32_t)per_cu, std::memory_order_relaxed);
-    return (uint32_t)per_cu;
-}
 // plan index of the few-row kernel (gemm_rows.h): 16 * MA activation rows,
 // 16 W rows per workgroup, at most SEG (nb) K segments of 512 per wave
 constexpr int kGemmSkinny = kGemmNumTiles;
@@ -1245,32 +1230,11 @@ struct GemmPlan {
 };
 
 
-// The K pipeline for a grid of one round of one workgroup per CU: 4 stages
-// for 32x128 and 64x128, 3 for 128x128; 256x128, whose pipelined K loop
-// already reads the next step under this step's MFMAs, keeps double
-// buffering (14336x4096 at M = 512: 25.4 vs 29.2 us with 3 stages); 256x256
-// has one.  (128x128 alone measured about 6 % faster double-buffered, but
-// 3 stages inside the 8B layer sequence of the config-5 stack: 3518-3530 vs
-// 3593-3614 us, same process.)
-int gemm_deep_stages(int tile) { return tile == 3 || tile == 4 ? 4 : tile == 2 ? 3 : 2; }
-
 // The few-row kernel: at most 64 activation rows, K a multiple of 512 in at
 // most 8 waves of up to 4 segments (2 for 64 rows).
 bool gemm_skinny_ok(uint32_t m, uint32_t k)
 {
     return m <= 64u && k % 512u == 0u && k / 512u <= (m <= 32u ? 32u : 16u);
-}
-// Measured on MI355X at m = 32 (us, HIP events; few-row kernel with 1 / 2 / 4
-// W fragments per workgroup, then the tiled 32x128): 4096x4096 5.81 / 6.62 /
-// 9.11, 10.11; 6144x4096 7.87 / 6.93 / 9.20, 11.60; 28672x4096 23.91 / 20.25
-// / 17.70, 21.49; 4096x14336 11.66 (one fragment), 15.35; 128256x4096 91.74
-// / 69.10 / 62.66, 68.67.  At m = 16 the 128256x4096 LM head 56.90 (4
-// fragments) against 64.78 tiled.  The few-row kernel wins at every shape up
-// to 32 rows.
-bool gemm_skinny_pays(uint32_t m, uint32_t n, uint32_t k)
-{
-    (void)n;
-    return gemm_skinny_ok(m, k) && m <= 32u;
 }
 // K segments per wave: the K segments over at most 8 waves
 uint32_t gemm_rows_seg(uint32_t k) { return k / 512u <= 8u ? 1u : (k / 512u <= 16u ? 2u : 4u); }
@@ -1293,130 +1257,161 @@ int gemm_rows_nf(int mb, int seg, uint32_t n, uint32_t num_cus)
 
 uint32_t ceil_div(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
-// Tile: the largest one that does not waste more than a quarter of its rows
-// on m and still yields a tile per CU; else the smallest such tile, with the
-// K split raised until every CU has a workgroup (bounded by the workspace).
-// Two measured exceptions below: 256x256 at 7/8 fill, and long K split in two.
-static GemmPlan gemm_plan_tile(uint32_t m, uint32_t n, uint32_t k, uint32_t num_cus)
+// Estimated time (us) of each compiled tiled kernel: with W workgroups (tiles
+// x K splits) of S K steps on C CUs, q = ceil(W / C) per CU and r = ceil(q /
+// occ) rounds of resident ones,
+//   t = 2 + r (fr + S sr) + q (fq + S sq) + W / C S sw  (+ the K split's sum),
+// joined (fourth-power mean) with the time to stream the weights at 5 TB/s.  r's
+// terms are a round's latencies, q's what a CU's workgroups share, the last
+// what the device shares.  Fitted to 21000 timings on MI355X (49
+// weight shapes of 512 .. 28672 rows and K 1024 .. 14336 at 8 to 2048
+// activation rows, and 413 random shapes; every compiled kernel, up to 8
+// splits, weights from HBM).  Past 32 rows the least estimate is within 1.2 %
+// (geometric mean; random shapes 1.9 %) of the fastest measured plan; the tile
+// thresholds used before were 18 % off it (2048x2048 at 48 rows split 8 ways
+// 9.9 us, 5.0 now; 11264x2048 at 320 rows 17.4, 9.7; 14336x4096 at 128 rows
+// 18.0, 12.5).
+struct GemmCost {
+    int tile, nst;
+    uint32_t occ;                 // workgroups per CU (registers and LDS of the compiled kernel)
+    float fr, sr, fq, sq, sw, c2; // c2: the in-launch sum of two K splits (256x256: by the reduce kernel)
+};
+constexpr GemmCost kGemmCost[] = {
+    {0, 2, 1, 3.681f, 0.511f, 3.931f, 0.566f, 1.246f, 3.000f},
+    {1, 2, 1, 2.299f, 0.240f, 3.245f, 0.449f, 0.515f, 6.778f},
+    {1, 3, 1, 4.224f, 0.513f, 3.164f, 0.211f, 0.415f, 6.846f},
+    {2, 2, 1, 1.296f, 0.326f, 1.293f, 0.199f, 0.336f, 4.643f},
+    {2, 3, 1, 2.009f, 0.314f, 2.198f, 0.156f, 0.183f, 4.552f},
+    {3, 2, 2, 0.991f, 0.426f, 0.421f, 0.050f, 0.183f, 2.965f},
+    {3, 3, 2, 2.013f, 0.158f, 0.411f, 0.208f, 0.104f, 2.920f},
+    {3, 4, 1, 2.062f, 0.162f, 0.563f, 0.146f, 0.127f, 2.826f},
+    {4, 2, 3, 0.637f, 0.381f, 0.080f, 0.063f, 0.111f, 2.054f},
+    {4, 4, 1, 0.573f, 0.025f, 1.225f, 0.225f, 0.082f, 1.933f},
+};
+
+float gemm_cost(const GemmCost &c, uint32_t kz, uint32_t m, uint32_t n, uint32_t k, uint32_t cus)
 {
-    const uint32_t nsuper = k / 256u;
-    if (t_gemm_tile == kGemmSkinny || (t_gemm_tile < 0 && gemm_skinny_pays(m, n, k))) {
-        // few activation rows: stream W like a GEMV, 16 NF W rows per
-        // workgroup (kz: NF, a forced plan may set it)
-        GemmPlan p{kGemmSkinny, 1u};
-        p.ma = m <= 16u ? 1 : (m <= 32u ? 2 : 4);
-        p.nb = (int)gemm_rows_seg(k);
-        p.kz = t_gemm_tile == kGemmSkinny && t_gemm_kz > 0 ? (uint32_t)t_gemm_kz
-                                                            : (uint32_t)gemm_rows_nf(p.ma, p.nb, n, num_cus);
-        return p;
-    }
-    int pick = t_gemm_tile;
-    if (pick < 0 && m >= 1024u) {
-        // many rows: the fewest rounds of resident workgroups (tiles over
-        // occupancy x CUs), then the fullest last round, then the most
-        // workgroups per CU.  Measured at M = 2048 (8B prefill): q|k|v 256x256
-        // 49.6 us (vs 60.0 for 256x128), o and down 128x128 29.6 / 82.2 us (vs
-        // 33.2 / 90.2), gate|up 256x256.
-        int best = -1;
-        uint64_t best_rounds = 0;
-        double best_fill = 0.0;
-        for (int i = 0; i < kGemmNumTiles; i++) {
-            const GemmTile &t = kGemmTiles[i];
-            if ((uint64_t)ceil_div(m, t.bm) * t.bm * 4u > (uint64_t)m * 5u) continue; // > 25% padding
-            const uint64_t nt = (uint64_t)ceil_div(m, t.bm) * ceil_div(n, t.bn), slots = (uint64_t)gemm_occ(i) * num_cus;
-            const uint64_t rounds = (nt + slots - 1) / slots;
-            const double fill = (double)nt / (double)(rounds * slots);
-            const bool better = best < 0 || rounds < best_rounds ||
-                                (rounds == best_rounds && (fill > best_fill + 0.01 ||
-                                                           (fill > best_fill - 0.01 && gemm_occ(i) > gemm_occ(best))));
-            if (better) best = i, best_rounds = rounds, best_fill = fill;
-        }
-        // (a grid under half the CUs goes to the K-split rule below)
-        if (best >= 0 && 2ull * ceil_div(m, kGemmTiles[best].bm) * ceil_div(n, kGemmTiles[best].bn) >= num_cus)
-            return {best, 1u};
-    }
-    if (pick < 0) {
-        // one round of 256x256 tiles over at least 7/8 of the CUs beats two
-        // rounds of 256x128 (one workgroup per CU either way): 8B gate|up at
-        // M = 512 (224 tiles) 50 vs 66 us
-        const GemmTile &t = kGemmTiles[0];
-        const uint64_t nt = (uint64_t)ceil_div(m, t.bm) * ceil_div(n, t.bn);
-        if ((uint64_t)ceil_div(m, t.bm) * t.bm * 4u <= (uint64_t)m * 5u && nt * 8u >= 7ull * num_cus && nt < num_cus)
-            return {0, 1u};
-        // likewise one round of 256x128 tiles over two rounds of 128x128:
-        // 14336x4096 at M = 512 25.4 us (double-buffered, pipelined loop)
-        // against 32.8; 28672x4096 at M = 256 26.4 against 34.0
-        const GemmTile &t1 = kGemmTiles[1];
-        const uint64_t nt1 = (uint64_t)ceil_div(m, t1.bm) * ceil_div(n, t1.bn);
-        if ((uint64_t)ceil_div(m, t1.bm) * t1.bm * 4u <= (uint64_t)m * 5u && nt1 * 8u >= 7ull * num_cus && nt1 < num_cus)
-            return {1, 1u};
-        // and one round of 128x128 tiles over at least 3/4 of the CUs over
-        // 64x128 tiles past one per CU: alone about equal (6144x4096 at M =
-        // 512 15.9-16.2 vs 14.9-15.2 us), but inside the 8B layer sequence
-        // of the config-5 stack the q|k|v shape on 128x128 saves about 2 us
-        // per layer (stack 3587 vs 3656-3670 us, same process)
-        const GemmTile &t2 = kGemmTiles[2];
-        const uint64_t nt2 = (uint64_t)ceil_div(m, t2.bm) * ceil_div(n, t2.bn);
-        if ((uint64_t)ceil_div(m, t2.bm) * t2.bm * 4u <= (uint64_t)m * 5u && nt2 * 4u >= 3ull * num_cus && nt2 < num_cus)
-            return {2, 1u};
-    }
-    for (int i = 0; pick < 0 && i < kGemmNumTiles; i++) {
-        const GemmTile &t = kGemmTiles[i];
-        if (t.bm > 32u && (uint64_t)ceil_div(m, t.bm) * t.bm * 4u > (uint64_t)m * 5u) continue; // > 25% padding
-        if ((uint64_t)ceil_div(m, t.bm) * ceil_div(n, t.bn) >= num_cus || i == kGemmNumTiles - 1) pick = i;
-    }
-    const uint64_t tiles = (uint64_t)ceil_div(m, kGemmTiles[pick].bm) * ceil_div(n, kGemmTiles[pick].bn);
-    if (t_gemm_kz > 0) return {pick, std::min<uint32_t>((uint32_t)t_gemm_kz, nsuper)};
-    if (tiles >= num_cus) {
-        // long K at about one workgroup per CU: two K splits let two
-        // workgroups per CU overlap their serial chains of K steps (8B down
-        // at M = 512: 64x128, 56 steps, 51 -> 37 us before the pipelined
-        // loop), if the workspace holds them
-        if (nsuper >= 32u && tiles < 2ull * num_cus && 2ull * m * n <= kGemmPartFloats) {
-            // or the next tile up in two splits as one round with a deeper
-            // pipeline (8B down at M = 512: 128x128 in two splits, 3 stages,
-            // 35.5 us against 48-50 for 64x128 in two before the pipelined
-            // loop; since, alone, 29-33 us against 28 for 64x128 unsplit with
-            // 4 stages, but inside the config-5 stack's layer sequence the
-            // split plan stays ahead)
-            const GemmTile &u = kGemmTiles[2];
-            const uint64_t tu = (uint64_t)ceil_div(m, u.bm) * ceil_div(n, u.bn);
-            if (pick == 3 && (uint64_t)ceil_div(m, u.bm) * u.bm * 4u <= (uint64_t)m * 5u && 2u * tu <= num_cus &&
-                8u * 2u * tu >= 7ull * num_cus)
-                return {2, 2u};
-            return {pick, 2u};
-        }
-        return {pick, 1u};
-    }
-    // short K over at least half the CUs: no split either (its partial sums
-    // cost more than the idle CUs: 6144x4096 at M = 128, 192 tiles of 32x128,
-    // 8.2 vs 11.1 us split in two; 4096x4096 at M = 128, 128 tiles, 8.0 vs
-    // 9.9; 8B gate|up at M = 32, 224 tiles, 17.0 vs 19.7)
-    if (nsuper < 32u && 2u * tiles >= num_cus) return {pick, 1u};
-    if (tiles * 8u >= 7ull * num_cus) return {pick, 1u};
-    // steps per split: as few as reach one workgroup per CU; kz = ceil(nsuper / per) leaves no split empty
-    uint32_t per = std::max<uint32_t>(1u, nsuper / ceil_div(num_cus, tiles));
-    uint32_t kz = ceil_div(nsuper, per);
-    while (kz > 1 && (uint64_t)kz * m * n > kGemmPartFloats) kz = ceil_div(nsuper, ++per);
-    return {pick, kz};
+    const GemmTile &t = kGemmTiles[c.tile];
+    const uint64_t w = (uint64_t)ceil_div(m, t.bm) * ceil_div(n, t.bn) * kz;
+    const float q = (float)((w + cus - 1u) / cus), r = (float)(((w + cus - 1u) / cus + c.occ - 1u) / c.occ);
+    const float s = (float)ceil_div(k / 256u, kz), mb = (float)m * (float)n * 4e-6f;
+    float us = 2.0f + r * (c.fr + s * c.sr) + q * (c.fq + s * c.sq) + (float)w / (float)cus * s * c.sw;
+    if (kz == 2u && c.tile > 0) us += c.c2 + 0.4f * mb;
+    else if (kz > 1u) us += 2.5f + 0.5f * (float)kz + 0.2f * (float)(kz + 1u) * mb; // the reduce kernel
+    const float hbm = 2.0f + (float)n * (float)k * (17.0f / 32.0f / 5.0e6f);
+    return std::sqrt(std::sqrt(us * us * us * us + hbm * hbm * hbm * hbm));
 }
 
-// The tile and K split, then the K pipeline: where the grid is one round of
-// one workgroup per CU (tiles x splits <= CUs), the deepest compiled one;
-// else double buffering (a deeper ring leaves fewer workgroups per CU).
-// Measured at M = 512 (us, 2 / 3 / 4 stages): 4096x4096 64x128 17.5 / 14.4
-// / 13.9; 1024x4096 32x128 in two splits 12.2 / - / 10.9; 6144x4096 64x128
-// (384 tiles) 19.6 / 21.4 / 24.6; 14336x4096 128x128 (448 tiles) 36.2 /
-// 39.5; 4096x14336 128x128 in two splits 45.3 / 35.5.  Same MFMA sequence at
-// any depth: bit-identical outputs.
-GemmPlan gemm_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t num_cus)
+// Whether kind's epilogue is compiled for (tile, nst) without a K split.
+bool gemm_kind_has(GemmKind kind, int tile, int nst)
 {
-    GemmPlan p = gemm_plan_tile(m, n, k, num_cus);
-    if (p.tile == kGemmSkinny) return p;
-    const uint64_t grid = (uint64_t)ceil_div(m, kGemmTiles[p.tile].bm) * ceil_div(n, kGemmTiles[p.tile].bn) * p.kz;
-    p.nst = grid <= num_cus ? gemm_deep_stages(p.tile) : 2;
-    if (t_gemm_stages) p.nst = t_gemm_stages;
+    if (kind == GEMM_ROPE)
+        return tile == 0 || (tile >= 2 && (nst == 2 || (nst == 3 && tile <= 3) || (nst == 4 && tile >= 3)));
+    if (kind == GEMM_SWIGLU) return tile == 0 || (tile == 2 && nst <= 3);
+    return true;
+}
+
+// The cheapest tiled plan.  A forced tile or split (test hooks) is taken as it
+// is.  fp4_gemm covers the CUs (7/8 of them, 3/4 by tiles of 128x128 or more;
+// half with a short K or from 1024 rows on) by K splits where the splits fit
+// the workspace, and pads rows by at most a quarter; the prefill's projections
+// are free of that.
+GemmPlan gemm_plan_tiles(uint32_t m, uint32_t n, uint32_t k, uint32_t cus, GemmKind kind)
+{
+    const uint32_t nsuper = k / 256u;
+    const bool split_ok = kind == GEMM_CALL || kind == GEMM_LAYER;
+    if (kind == GEMM_CALL && t_gemm_tile < 0 && !t_gemm_kz && !t_gemm_stages && nsuper >= 32u && m < 1024u) {
+        // long K, 128x128 tiles over about half the CUs: two splits as one
+        // round.  Alone 64x128 unsplit with 4 stages is faster (4096x14336 at
+        // M = 512 28-30 against 31-32 us), inside a layer's sequence of calls
+        // the split plan was.
+        const GemmTile &u = kGemmTiles[2];
+        const uint64_t tu = (uint64_t)ceil_div(m, u.bm) * ceil_div(n, u.bn);
+        if ((uint64_t)ceil_div(m, u.bm) * u.bm * 4u <= (uint64_t)m * 5u && 2u * tu <= cus && 16u * tu >= 7ull * cus &&
+            2ull * m * n <= kGemmPartFloats)
+            return {2, 2u, 0, 0, 3};
+    }
+    const uint32_t cover = m >= 1024u || nsuper < 32u ? cus / 2u : cus * 7u / 8u;
+    for (int pass = 0; pass < 2; pass++) { // pass 1: no plan covers the CUs
+        GemmPlan best{-1, 1u};
+        float least = 0.0f;
+        for (const GemmCost &c : kGemmCost) {
+            const GemmTile &t = kGemmTiles[c.tile];
+            if (t_gemm_tile >= 0 && c.tile != t_gemm_tile) continue;
+            if (t_gemm_stages && c.tile > 0 && c.nst != t_gemm_stages) continue;
+            if (!gemm_kind_has(kind, c.tile, c.nst)) continue;
+            const uint64_t tiles = (uint64_t)ceil_div(m, t.bm) * ceil_div(n, t.bn);
+            if (kind == GEMM_CALL && t_gemm_tile < 0 && t.bm > 32u && (uint64_t)ceil_div(m, t.bm) * t.bm * 4u > (uint64_t)m * 5u)
+                continue;
+            const uint32_t kz_max = t_gemm_kz > 0 ? std::min<uint32_t>((uint32_t)t_gemm_kz, nsuper)
+                                                  : split_ok ? std::min(8u, nsuper) : 1u;
+            for (uint32_t kz = t_gemm_kz > 0 ? kz_max : 1u; kz <= kz_max; kz++) {
+                const uint32_t per = ceil_div(nsuper, kz);
+                if (!t_gemm_kz && ((uint64_t)(kz - 1u) * per >= nsuper || (kz > 1u && (uint64_t)kz * m * n > kGemmPartFloats)))
+                    continue; // an empty split, or past the workspace
+                const bool covered = tiles * kz >= cover || (c.tile <= 2 && tiles * 4u >= 3ull * cus);
+                if (pass == 0 && kind == GEMM_CALL && t_gemm_tile < 0 && !t_gemm_kz && !covered && kz != nsuper &&
+                    (uint64_t)(kz + 1u) * m * n <= kGemmPartFloats)
+                    continue;
+                const float us = gemm_cost(c, kz, m, n, k, cus);
+                if (best.tile < 0 || us < least) best = GemmPlan{c.tile, kz, 0, 0, c.nst}, least = us;
+            }
+        }
+        if (best.tile >= 0) return best;
+    }
+    // a forced stage count that no candidate has: the launch names the kernel that is missing
+    return {t_gemm_tile >= 0 ? t_gemm_tile : 2, t_gemm_kz > 0 ? std::min<uint32_t>((uint32_t)t_gemm_kz, nsuper) : 1u, 0, 0,
+            t_gemm_stages ? t_gemm_stages : 2};
+}
+
+// The few-row kernel streams W like a GEMV, one workgroup per 16 NF rows over
+// all of K.  fp4_gemm takes it up to 32 rows.  From 33 to 64 rows, and in the
+// prefill, where one round of workgroups of one or (to 32 rows, K up to 8192)
+// two W fragments holds the matrix: measured (us, few-row / best tiled)
+// 4096x4096 at 8, 32, 64 rows 5.2 / 7.7, 5.8 / 7.9, 7.3 / 8.2; 6144x4096 at
+// 32, 64 rows 6.9 / 8.1, 8.3 / 8.3; 11264x4096 at 32 rows 10.2 / 9.8;
+// 2048x8192 at 64 rows 10.2 / 10.0.
+bool gemm_rows_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t cus, GemmKind kind, GemmPlan *p)
+{
+    if (t_gemm_tile >= 0 ? t_gemm_tile != kGemmSkinny : (!gemm_skinny_ok(m, k) || kind == GEMM_ROPE || kind == GEMM_SWIGLU))
+        return false;
+    p->tile = kGemmSkinny;
+    p->ma = m <= 16u ? 1 : (m <= 32u ? 2 : 4);
+    p->nb = (int)gemm_rows_seg(k);
+    if (t_gemm_tile == kGemmSkinny || (kind == GEMM_CALL && m <= 32u)) {
+        p->kz = t_gemm_tile == kGemmSkinny && t_gemm_kz > 0 ? (uint32_t)t_gemm_kz : (uint32_t)gemm_rows_nf(p->ma, p->nb, n, cus);
+        return true;
+    }
+    if (n <= 16u * cus) p->kz = 1u;
+    else if (m <= 32u && n <= 32u * cus && gemm_rows_has(p->ma, p->nb, 2)) p->kz = 2u;
+    else return false;
+    return true;
+}
+
+// The plan: a function of its arguments (and this thread's test hooks) alone,
+// remembered per thread for the last shapes asked, since it tries up to 80
+// candidates (about 1.5 us).
+GemmPlan gemm_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t num_cus, GemmKind kind = GEMM_CALL)
+{
+    struct Entry {
+        uint32_t m, n, k, cus, kind;
+        GemmPlan p;
+    };
+    static thread_local Entry seen[64] = {};
+    const bool hooked = t_gemm_tile >= 0 || t_gemm_kz || t_gemm_stages;
+    Entry &e = seen[(m * 31u + n * 7u + k / 256u + (uint32_t)kind * 13u) % 64u];
+    if (!hooked && e.m == m && e.n == n && e.k == k && e.cus == num_cus && e.kind == (uint32_t)kind) return e.p;
+    GemmPlan p{};
+    if (!gemm_rows_plan(m, n, k, num_cus, kind, &p)) p = gemm_plan_tiles(m, n, k, num_cus, kind);
+    if (!hooked) e = Entry{m, n, k, num_cus, (uint32_t)kind, p};
     return p;
+}
+
+float gemm_plan_cost(const GemmPlan &p, uint32_t m, uint32_t n, uint32_t k, uint32_t cus)
+{
+    for (const GemmCost &c : kGemmCost)
+        if (c.tile == p.tile && c.nst == p.nst) return gemm_cost(c, p.kz, m, n, k, cus);
+    return 0.0f; // the few-row kernel
 }
 
 // The 8-wave ping-pong kernel (rfp4_gemm_<tile>_pp) for a plan of the
@@ -1463,13 +1458,13 @@ bool gemm_accumulate_ok(uint32_t m, uint32_t n, uint32_t k)
 {
     Runtime *rt = g_rt;
     if (!rt || !m || !n || !k || k % 256u) return false;
-    const GemmPlan p = gemm_plan(m, n, k, (uint32_t)rt->num_cus);
+    const GemmPlan p = gemm_plan(m, n, k, (uint32_t)rt->num_cus, GEMM_LAYER);
     return p.tile != kGemmSkinny && (p.tile != 0 || gemm_use_pp(p, m, n, k));
 }
 
 int gemm_launch(hipStream_t stream, uint32_t m, uint32_t n, uint32_t k, const uint8_t *a_codes, const uint8_t *a_scales,
                 const uint8_t *a_st, const uint8_t *w_codes, const uint8_t *w_scales, const uint8_t *w_st, float *c,
-                float *part, bool accumulate)
+                float *part, bool accumulate, GemmKind kind)
 {
     if (!a_codes || !a_scales || !w_codes || !w_scales || !c) return set_error(RFP4_E_INVALID, "fp4_gemm: null pointer");
     if (m == 0 || n == 0 || k == 0) return set_error(RFP4_E_SHAPE, "fp4_gemm: empty shape m=%u n=%u k=%u", m, n, k);
@@ -1481,7 +1476,7 @@ int gemm_launch(hipStream_t stream, uint32_t m, uint32_t n, uint32_t k, const ui
         return set_error(RFP4_E_ALIGN, "fp4_gemm: scales must be 8-byte aligned");
     Runtime *rt = g_rt;
     if (!rt) return set_error(RFP4_E_NOT_INIT, "rfp4_init has not been called");
-    GemmPlan p = gemm_plan(m, n, k, (uint32_t)rt->num_cus);
+    GemmPlan p = gemm_plan(m, n, k, (uint32_t)rt->num_cus, kind);
     if (p.tile == kGemmSkinny) {
         if (accumulate) return set_error(RFP4_E_INVALID, "fp4_gemm: no accumulating few-row kernel (m=%u)", m);
         if (!gemm_skinny_ok(m, k))
@@ -1540,17 +1535,26 @@ int gemm_launch(hipStream_t stream, uint32_t m, uint32_t n, uint32_t k, const ui
                   (hipStream_t)stream, &a);
 }
 
-// The kernel with the SwiGLU epilogue for the plan of the plain GEMM (m, 2
-// ffn, k), no K split: the 256x256 ping-pong tile (ffn % 256 == 0: whole
-// 128-column pairs and step-blocked output scales), or the 128x128 tile with
-// 2 or 3 stages (64-column pairs).  Null: none.
+// The kernel with the SwiGLU epilogue for the plan of (m, 2 ffn, k): the
+// 256x256 ping-pong tile (ffn % 256 == 0: whole 128-column pairs and
+// step-blocked output scales), or the 128x128 tile with 2 or 3 stages
+// (64-column pairs).  Null: none, or the plain GEMM's best plan and the row
+// kernel (about 3 us and the f32 gate|up rows there and back) take less:
+// measured so at 48 rows of TinyLlama (10.6 us against 11.6), not from 128 rows
+// on (11.0 against 12.2; Llama-3-8B at 200 rows 30.4 against 35.5).
 static const char *gemm_swiglu_kernel(uint32_t m, uint32_t ffn, uint32_t k, uint32_t &cols)
 {
     Runtime *rt = g_rt;
     if (!rt || m == 0 || ffn == 0 || ffn % 256u || k == 0 || k % 256u) return nullptr;
-    const GemmPlan p = gemm_plan(m, 2u * ffn, k, (uint32_t)rt->num_cus);
+    const uint32_t cus = (uint32_t)rt->num_cus;
+    const GemmPlan p = gemm_plan(m, 2u * ffn, k, cus, GEMM_SWIGLU);
     if (p.kz != 1u) return nullptr;
     const bool pp = gemm_use_pp(p, m, 2u * ffn, k);
+    if (t_gemm_tile < 0 && !t_gemm_stages) {
+        const GemmPlan plain = gemm_plan(m, 2u * ffn, k, cus, GEMM_LAYER);
+        const float rows = 3.0f + (float)m * (float)ffn * (16.0f / 4.0e6f);
+        if (gemm_plan_cost(p, m, 2u * ffn, k, cus) > gemm_plan_cost(plain, m, 2u * ffn, k, cus) + rows) return nullptr;
+    }
     if (p.tile == 0 && pp) {
         cols = 128u;
         return "rfp4_gemm_256x256_ppsw";
@@ -1600,7 +1604,7 @@ static bool gemm_rope_kernel(uint32_t m, uint32_t n, uint32_t k, RopeKernel &rk)
 {
     Runtime *rt = g_rt;
     if (!rt || m == 0 || n == 0 || k == 0 || k % 256u) return false;
-    const GemmPlan p = gemm_plan(m, n, k, (uint32_t)rt->num_cus);
+    const GemmPlan p = gemm_plan(m, n, k, (uint32_t)rt->num_cus, GEMM_ROPE);
     if (p.tile == kGemmSkinny || p.kz != 1u) return false;
     const bool pp = gemm_use_pp(p, m, n, k);
     rk.tile = p.tile;

@@ -91,6 +91,12 @@ size_t engines_destroy_all();
 // Looks up, once per device and with that device current, the address of
 // the allocation-free entry points' static scratch (csrc/noalloc.hip).
 int noalloc_setup(int device);
+// Who plans a GEMM.  GEMM_CALL: fp4_gemm and fp4_gemm_tiled.  GEMM_LAYER: the
+// prefill's projections.  GEMM_ROPE and GEMM_SWIGLU: its q|k|v and gate|up
+// projections where their epilogues are used, which exist for some kernels
+// without a K split; planned the same whether the epilogue or the row kernel
+// after the GEMM does that work, so that the sums agree.
+enum GemmKind { GEMM_CALL, GEMM_LAYER, GEMM_ROPE, GEMM_SWIGLU };
 // fp4_gemm with the caller's split-K workspace (kGemmWorkspaceWords words, the
 // counters zeroed; the engine owns one, so engines on different streams do
 // not share partials).  a_st / w_st: the step-blocked copies of the scales
@@ -101,14 +107,15 @@ int noalloc_setup(int device);
 // (gemm_accumulate_ok).
 int gemm_launch(hipStream_t stream, uint32_t m, uint32_t n, uint32_t k, const uint8_t *a_codes, const uint8_t *a_scales,
                 const uint8_t *a_st, const uint8_t *w_codes, const uint8_t *w_scales, const uint8_t *w_st, float *c,
-                float *part, bool accumulate = false);
-bool gemm_accumulate_ok(uint32_t m, uint32_t n, uint32_t k);
+                float *part, bool accumulate = false, GemmKind kind = GEMM_CALL);
+bool gemm_accumulate_ok(uint32_t m, uint32_t n, uint32_t k); // of the GEMM_LAYER plan
 // The gate|up projection of the prefill with SwiGLU and the MXFP4 rows of its
 // output in the GEMM's epilogue (rfp4_gemm_256x256_ppsw): m rows of K = k,
 // W = [gate; up] of 2 ffn rows; y = silu(gate) * up quantized per 32 into
 // q_codes [m][ffn/2], q_scales [m][ffn/32] and q_scales_t (step-blocked).
-// gemm_swiglu_ok: whether the plan of the plain GEMM (m, 2 ffn, k) is that
-// kernel's tile (256x256 ping-pong, no K split) and ffn a multiple of 256.
+// gemm_swiglu_ok: whether the GEMM_SWIGLU plan of (m, 2 ffn, k) has that
+// epilogue, ffn is a multiple of 256, and it is estimated to take less than
+// the plain GEMM and the row kernel.
 bool gemm_swiglu_ok(uint32_t m, uint32_t ffn, uint32_t k);
 int gemm_swiglu_launch(hipStream_t stream, uint32_t m, uint32_t ffn, uint32_t k, const uint8_t *a_codes,
                        const uint8_t *a_scales, const uint8_t *a_st, const uint8_t *w_codes, const uint8_t *w_scales,
@@ -117,10 +124,9 @@ int gemm_swiglu_launch(hipStream_t stream, uint32_t m, uint32_t ffn, uint32_t k,
 // the GEMM's epilogue (the _rope kernels; GemmArgs::rope_cos): m rows of
 // K = k into n = q + 2 kv columns of c, heads hd wide, row r at position
 // pos0 + r, cache element (pos, kv head, d) at pos * ts + head * hs + d.
-// gemm_rope_ok: whether the plan of the plain GEMM (m, n, k) is a tile with
-// that epilogue compiled (128x128 with 2 or 3 stages, 256x256 ping-pong; no
-// K split) and hd 64 or 128; its output is then bit-identical to the GEMM
-// followed by the RoPE + K/V row kernel.
+// gemm_rope_ok: whether the GEMM_ROPE plan of (m, n, k) has that epilogue
+// compiled and hd is 64 or 128; its output is then bit-identical to that
+// plan's GEMM followed by the RoPE + K/V row kernel.
 struct GemmRope {
     const float *cosv, *sinv;
     uint16_t *kc, *vc;
