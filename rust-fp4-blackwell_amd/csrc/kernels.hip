@@ -273,13 +273,15 @@ K256 void rfp4_scales_tile(ScaleTileArgs a) { scales_tile_body(a); }
 // few activation rows (M <= 16 MB) x 16 NF W rows per workgroup, up to 8
 // waves of up to SEG K segments of 512 each (device/gemm_rows.h):
 // rfp4_gemm_rows_m<16 MB>_s<SEG>_f<NF>, the combinations whose loads fit the
-// registers (runtime.cpp gemm_rows_has); keep the two lists in sync.
+// registers (runtime.cpp gemm_rows_has); keep the two lists in sync.  _f4: a
+// wave per fragment of all K, two waves per SIMD (a fragment in registers).
 #define GEMM_ROWS_KERNEL(M, MB, SEG, NF) \
     K512 void rfp4_gemm_rows_m##M##_s##SEG##_f##NF(GemmArgs a) { gemm_rows_body<MB, SEG, NF>(a); }
 #define GEMM_ROWS_SMALL_M(M, MB) \
     GEMM_ROWS_KERNEL(M, MB, 1, 1) \
     GEMM_ROWS_KERNEL(M, MB, 1, 2) \
-    GEMM_ROWS_KERNEL(M, MB, 1, 4) \
+    extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void \
+        rfp4_gemm_rows_m##M##_s1_f4(GemmArgs a) { gemm_rows_wide_body<MB>(a); } \
     GEMM_ROWS_KERNEL(M, MB, 2, 1) \
     GEMM_ROWS_KERNEL(M, MB, 2, 2) \
     GEMM_ROWS_KERNEL(M, MB, 4, 1)

@@ -1486,9 +1486,16 @@ int gemm_launch(hipStream_t stream, uint32_t m, uint32_t n, uint32_t k, const ui
             return set_error(RFP4_E_INVALID, "fp4_gemm: no few-row variant with %d W fragments for m=%u k=%u", (int)p.kz, m, k);
         char name[48];
         snprintf(name, sizeof name, "rfp4_gemm_rows_m%d_s%d_f%u", 16 * p.ma, p.nb, p.kz);
-        const uint32_t waves = ceil_div(k / 512u, (uint32_t)p.nb);
-        GemmArgs a{a_codes, a_scales, w_codes, w_scales, c, nullptr, m, n, k, 1u};
-        return launch(name, dim3(ceil_div(n, 16u * p.kz)), dim3(64u * waves), (hipStream_t)stream, &a);
+        uint32_t waves = ceil_div(k / 512u, (uint32_t)p.nb), grid = ceil_div(n, 16u * p.kz);
+        if (p.kz == 4u) {
+            // a wave per fragment of 16 rows: one workgroup per CU, the waves
+            // (at most 8) that spread the fragments evenly in the fewest rounds
+            const uint32_t frags = ceil_div(n, 16u), cus = (uint32_t)rt->num_cus;
+            waves = ceil_div(frags, cus * ceil_div(frags, 8u * cus));
+            grid = std::min(ceil_div(frags, waves), cus);
+        }
+        GemmArgs a{a_codes, a_scales, w_codes, w_scales, c, nullptr, m, n, k, waves};
+        return launch(name, dim3(grid), dim3(64u * waves), (hipStream_t)stream, &a);
     }
     const GemmTile &t = kGemmTiles[p.tile];
     const uint64_t tiles = (uint64_t)ceil_div(m, t.bm) * ceil_div(n, t.bn);
