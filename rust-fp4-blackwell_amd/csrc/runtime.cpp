@@ -1186,7 +1186,7 @@ int mx4_quantize_st(hipStream_t stream, uint64_t rows, uint64_t k, const void *s
     if (((uintptr_t)src & (src_is_bf16 ? 7u : 15u)) != 0)
         return set_error(RFP4_E_ALIGN, "mx4_quantize: src must be %u-byte aligned", src_is_bf16 ? 8u : 16u);
     QuantMxArgs a{src, codes, scales, rows, k, scales_t};
-    uint64_t blocks = (rows * (k / 4) + 255) / 256; // one thread per 4 values
+    uint64_t blocks = (rows * (k / 8) + 255) / 256; // one thread per 8 values
     if (blocks > 65536) blocks = 65536;
     return launch(src_is_bf16 ? "rfp4_quant_mx_bf16" : "rfp4_quant_mx_f32", dim3((unsigned)blocks), dim3(256), stream, &a);
 }
