@@ -813,7 +813,7 @@ struct AttnSplit {
 
         if (nsplit == 1) {
             // one split holds the whole sequence: normalise and write the heads' outputs
-            for (uint32_t i = tid; i < G * HD; i += blockDim.x) {
+            for (uint32_t i = tid; i < G * HD; i += 256u) {
                 const uint32_t g = i / HD, d = i % HD;
                 const float v = vred[0][g][d] + vred[1][g][d] + vred[2][g][d] + vred[3][g][d];
                 const float l = (s_lred[0][g] + s_lred[1][g]) + (s_lred[2][g] + s_lred[3][g]);
@@ -829,7 +829,7 @@ struct AttnSplit {
         const uint32_t stride = HD + 4;
         if (TAG) {
             const uint32_t tag = seq;
-            for (uint32_t i = tid; i < G * HD; i += blockDim.x) {
+            for (uint32_t i = tid; i < G * HD; i += 256u) {
                 const uint32_t g = i / HD, d = i % HD;
                 const float v = vred[0][g][d] + vred[1][g][d] + vred[2][g][d] + vred[3][g][d];
                 const float l = (s_lred[0][g] + s_lred[1][g]) + (s_lred[2][g] + s_lred[3][g]);
@@ -846,7 +846,7 @@ struct AttnSplit {
             return;
         }
         const bool inmerge = a.counters != nullptr;
-        for (uint32_t i = tid; i < G * HD; i += blockDim.x) {
+        for (uint32_t i = tid; i < G * HD; i += 256u) {
             uint32_t g = i / HD, d = i % HD;
             float v = vred[0][g][d] + vred[1][g][d] + vred[2][g][d] + vred[3][g][d];
             size_t base = ((size_t)(hbase + g) * a.max_splits + split) * stride;

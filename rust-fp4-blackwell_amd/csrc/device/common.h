@@ -101,6 +101,32 @@ RFP4_DEV float wave_max(float v)
     return xor32_max(xor16_max(v));
 }
 
+// Largest 64-bit key over all 64 lanes, in every lane (the moves of wave_sum
+// on both halves of the key).
+template <int CTRL>
+RFP4_DEV unsigned long long dpp_max_u64(unsigned long long v)
+{
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, 0xF, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, 0xF, 0xF, false);
+    const unsigned long long o = ((unsigned long long)hi << 32) | lo;
+    return o > v ? o : v;
+}
+RFP4_DEV unsigned long long wave_max_u64(unsigned long long v)
+{
+    v = dpp_max_u64<DPP_QUAD_1032>(v);
+    v = dpp_max_u64<DPP_QUAD_2301>(v);
+    v = dpp_max_u64<DPP_ROW_HALF_MIRROR>(v);
+    v = dpp_max_u64<DPP_ROW_MIRROR>(v);
+    const auto l16 = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+    const auto h16 = __builtin_amdgcn_permlane16_swap((uint32_t)(v >> 32), (uint32_t)(v >> 32), false, false);
+    const unsigned long long a = ((unsigned long long)h16[0] << 32) | l16[0], b = ((unsigned long long)h16[1] << 32) | l16[1];
+    v = a > b ? a : b;
+    const auto l32 = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+    const auto h32 = __builtin_amdgcn_permlane32_swap((uint32_t)(v >> 32), (uint32_t)(v >> 32), false, false);
+    const unsigned long long c = ((unsigned long long)h32[0] << 32) | l32[0], d = ((unsigned long long)h32[1] << 32) | l32[1];
+    return c > d ? c : d;
+}
+
 // ---------------------------------------------------------------- fp16 matrix-core operands
 // v_mfma_f32_16x16x32_f16 operands: lane l holds A row / B column l % 16 and
 // K = 8 (l / 16) .. +7; accumulator r of lane l is D[4 (l / 16) + r][l % 16]

@@ -1162,7 +1162,7 @@ RFP4_DEV void gemm_pp_body(const GemmArgs &g)
 RFP4_DEV void gemm_reduce_body(const GemmArgs &g)
 {
     const size_t plane = (size_t)g.m * g.n, n4 = plane / 4u;
-    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n4; e += (size_t)gridDim.x * blockDim.x) {
+    for (size_t e = (size_t)blockIdx.x * 256u + threadIdx.x; e < n4; e += (size_t)gridDim.x * 256u) {
         float4 sum = ((const float4 *)g.part)[e];
         for (uint32_t z = 1; z < g.kz; z++) {
             const float4 p = ((const float4 *)(g.part + z * plane))[e];
@@ -1188,7 +1188,7 @@ RFP4_DEV void scales_tile_body(const ScaleTileArgs &a)
     const uint32_t nsuper = a.k >> 8, nblk = a.k >> 5;
     const uint64_t w0 = (uint64_t)((a.rows[0] + 31u) >> 5) * nsuper * 64u;
     const uint64_t words = w0 + (uint64_t)((a.rows[1] + 31u) >> 5) * nsuper * 64u;
-    for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < words; t += (uint64_t)gridDim.x * blockDim.x) {
+    for (uint64_t t = (uint64_t)blockIdx.x * 256u + threadIdx.x; t < words; t += (uint64_t)gridDim.x * 256u) {
         const uint32_t mtx = t < w0 ? 0u : 1u;
         const uint64_t w = t - (mtx ? w0 : 0u);
         const uint32_t l = (uint32_t)(w & 63u);

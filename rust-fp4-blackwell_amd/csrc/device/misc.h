@@ -6,8 +6,8 @@
 // ---------------------------------------------------------------- fill (memset replacement)
 RFP4_DEV void fill_body(const FillArgs &a)
 {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n_words;
-         i += (uint64_t)gridDim.x * blockDim.x)
+    for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < a.n_words;
+         i += (uint64_t)gridDim.x * 256u)
         a.p[i] = a.value;
 }
 
@@ -15,7 +15,7 @@ RFP4_DEV void fill_body(const FillArgs &a)
 template <int DST_F16>
 RFP4_DEV void copy_into_body(const CopyArgs &a)
 {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= a.n) return;
     if (DST_F16)
         ((uint16_t *)a.dst)[(size_t)a.off + i] = f32_to_f16_bits(a.src[i]);
@@ -26,7 +26,7 @@ RFP4_DEV void copy_into_body(const CopyArgs &a)
 // ---------------------------------------------------------------- swiglu / residual (llama_run/src/main.rs:244-261)
 RFP4_DEV void swiglu_body(const EltwiseArgs &a)
 {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= a.n) return;
     float g = a.a[i];
     float s = __fdiv_rn(g, __fadd_rn(1.0f, expf(-g)));
@@ -35,7 +35,7 @@ RFP4_DEV void swiglu_body(const EltwiseArgs &a)
 
 RFP4_DEV void residual_body(const EltwiseArgs &a)
 {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= a.n) return;
     a.out[i] = __fadd_rn(a.out[i], a.a[i]);
 }
@@ -47,90 +47,89 @@ RFP4_DEV void argmax_body(const ArgmaxArgs &a)
 {
     __shared__ unsigned long long red[16];
     unsigned long long best = pack_argmax(-1e30f, 0u);
-    for (uint32_t i = threadIdx.x; i < a.n; i += blockDim.x) {
+    for (uint32_t i = threadIdx.x; i < a.n; i += 1024u) {
         float v = a.logits[i];
         if (v > -1e30f) {
             unsigned long long k = pack_argmax(v, i);
             best = k > best ? k : best;
         }
     }
-    // wave reduce on the 64-bit key
-    for (int off = 32; off >= 1; off >>= 1) {
-        unsigned long long o = __shfl_xor(best, off, 64);
-        best = o > best ? o : best;
-    }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    best = wave_max_u64(best);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (lane == 0) red[wave] = best;
     __syncthreads();
     if (threadIdx.x == 0) {
         unsigned long long b = red[0];
-        for (int w = 1; w < nw; w++) b = red[w] > b ? red[w] : b;
+#pragma unroll
+        for (int w = 1; w < 16; w++) b = red[w] > b ? red[w] : b;
         *a.out = 0xFFFFFFFFu - (uint32_t)(b & 0xFFFFFFFFull);
     }
 }
 
 // The largest of n per-workgroup keys (one workgroup of 1024 threads): each
-// thread's loads of four keys issued together, then the wave and workgroup
-// reductions.  Thread 0 returns the maximum.
-RFP4_DEV unsigned long long keys_max(const unsigned long long *keys, uint32_t n)
+// thread's loads of four keys issued together, then the wave (keys_wave_max)
+// and workgroup (keys_block_max) reductions; every thread gets the maximum.
+RFP4_DEV unsigned long long keys_wave_max(const unsigned long long *keys, uint32_t n)
 {
-    __shared__ unsigned long long red[16];
     unsigned long long best = 0ull;
-    for (uint32_t i0 = threadIdx.x; i0 < n; i0 += 4u * blockDim.x) {
+    for (uint32_t i0 = threadIdx.x; i0 < n; i0 += 4096u) {
         unsigned long long v[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) v[j] = keys[min(i0 + (uint32_t)j * blockDim.x, n - 1u)];
+        for (int j = 0; j < 4; j++) v[j] = keys[min(i0 + (uint32_t)j * 1024u, n - 1u)];
 #pragma unroll
         for (int j = 0; j < 4; j++) best = v[j] > best ? v[j] : best;
     }
-    for (int off = 32; off >= 1; off >>= 1) {
-        unsigned long long o = __shfl_xor(best, off, 64);
-        best = o > best ? o : best;
-    }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    if (lane == 0) red[wave] = best;
+    return wave_max_u64(best);
+}
+
+RFP4_DEV unsigned long long keys_block_max(unsigned long long best)
+{
+    __shared__ unsigned long long red[16];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = best;
     __syncthreads();
     unsigned long long b = red[0];
-    for (int w = 1; w < nw; w++) b = red[w] > b ? red[w] : b;
+#pragma unroll
+    for (int w = 1; w < 16; w++) b = red[w] > b ? red[w] : b;
     return b;
 }
 
 // The token of an argmax GEMV's keys (ArgmaxKeysArgs): where no decode cursor
 // moves (mx4_gemv_argmax, the batched prefill's last row).  Latency bound
-// (4008 keys of a 128256-row head: 5.3 us in the trace, one launch instead of
+// (4008 keys of a 128256-row head: 4.5 us in the trace, one launch instead of
 // the 4.6 + 4.5 us of clearing a scratch cursor and running the step kernel;
 // the prefill ran the one-workgroup argmax over all logits, 49.7 us).
 RFP4_DEV void argmax_keys_body(const ArgmaxKeysArgs &a)
 {
-    const unsigned long long b = keys_max(a.best, a.n_best);
+    const unsigned long long b = keys_block_max(keys_wave_max(a.best, a.n_best));
     if (threadIdx.x == 0) *a.out = 0xFFFFFFFFu - (uint32_t)(b & 0xFFFFFFFFull);
 }
 
 // ---------------------------------------------------------------- end of decode step
+// Latency bound, a chain of dependent loads: the cursor and the prompt's next
+// token are fetched beside the keys, and every thread holds the token, so the
+// embedding row is the only load after the reduction (4008 keys: 5.4 -> 4.5 us).
 RFP4_DEV void step_body(const StepArgs &a)
 {
-    const unsigned long long b = keys_max(a.best, a.n_best);
-    __shared__ uint32_t s_next;
+    const int pos = a.state->pos, step = a.state->step;
+    const uint32_t n_prompt = a.state->n_prompt, ids_cap = a.state->ids_cap, nxt = (uint32_t)step + 1u;
+    const uint32_t given = nxt < n_prompt ? a.ids[nxt] : 0u;
+    const unsigned long long best = keys_wave_max(a.best, a.n_best);
+    // every wave has its cursor before the barrier that lets thread 0 move it
+    asm volatile("" ::"v"(pos), "v"(step), "v"(n_prompt), "v"(ids_cap), "v"(given));
+    const uint32_t tok = 0xFFFFFFFFu - (uint32_t)(keys_block_max(best) & 0xFFFFFFFFull);
     if (threadIdx.x == 0) {
-        uint32_t tok = 0xFFFFFFFFu - (uint32_t)(b & 0xFFFFFFFFull);
-        StepState st = *a.state;
         *a.last_tok = tok;
-        uint32_t nxt = (uint32_t)st.step + 1u;
-        if (nxt >= st.n_prompt && nxt < st.ids_cap) a.ids[nxt] = tok;
-        // the next step's input token: a prompt token, else this step's argmax
-        s_next = nxt < st.n_prompt ? a.ids[nxt] : tok;
-        st.step += 1;
-        st.pos += 1;
-        *a.state = st;
+        if (nxt >= n_prompt && nxt < ids_cap) a.ids[nxt] = tok;
+        a.state->step = step + 1;
+        a.state->pos = pos + 1;
     }
     if (!a.embed) return;
     // the next step's embedding (rfp4_embed's gather, done here so the step
-    // graph has one launch less)
-    __syncthreads();
-    uint32_t t = s_next;
+    // graph has one launch less): a prompt token, else this step's argmax
+    uint32_t t = nxt < n_prompt ? given : tok;
     if (t >= a.vocab) t = 0;
     const uint16_t *row = a.embed + (size_t)t * a.dim;
-    for (uint32_t i = threadIdx.x; i < a.dim; i += blockDim.x) a.x[i] = half_bits_to_f32(row[i], a.bf16 != 0);
+    for (uint32_t i = threadIdx.x; i < a.dim; i += 1024u) a.x[i] = half_bits_to_f32(row[i], a.bf16 != 0);
 }
 
 // ---------------------------------------------------------------- OCP MX block quantizer
@@ -243,7 +242,7 @@ RFP4_DEV void synth_weight_body(const SynthWeightArgs &a)
 {
     const uint64_t nb = a.k / 32;
     const uint64_t total = a.nrows * nb;
-    for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (uint64_t)gridDim.x * blockDim.x) {
+    for (uint64_t t = (uint64_t)blockIdx.x * 256u + threadIdx.x; t < total; t += (uint64_t)gridDim.x * 256u) {
         uint64_t rr = t / nb, blk = t % nb;
         uint64_t base = (a.r0 + rr) * a.k + blk * 32;
         float v[32];
@@ -256,7 +255,7 @@ RFP4_DEV void synth_weight_body(const SynthWeightArgs &a)
 
 RFP4_DEV void synth_f16_body(const SynthF16Args &a)
 {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += (uint64_t)gridDim.x * blockDim.x)
+    for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < a.n; i += (uint64_t)gridDim.x * 256u)
         a.out[i] = f32_to_f16_bits(__fadd_rn(a.offset, ih4_normal(mix64(a.seed, a.stream, i), a.coef)));
 }
 
@@ -264,7 +263,7 @@ RFP4_DEV void synth_f16_body(const SynthF16Args &a)
 RFP4_DEV void synth_kv_body(const SynthKvArgs &a)
 {
     const uint64_t total = (uint64_t)a.upto * a.n_kv_heads * a.head_dim;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (uint64_t)gridDim.x * blockDim.x) {
+    for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < total; i += (uint64_t)gridDim.x * 256u) {
         uint64_t d = i % a.head_dim, r = i / a.head_dim, kvh = r % a.n_kv_heads, t = r / a.n_kv_heads;
         float v = ih4_normal(mix64(a.seed, a.stream, i), a.coef);
         const uint64_t at = (kvh * a.max_seq + t) * a.head_dim + d;
@@ -345,7 +344,7 @@ RFP4_DEV void quant_mx_body(const QuantMxArgs &a)
 // (pins the builtin's nibble order against the host codec).
 RFP4_DEV void selftest_cvt_body(const SelftestArgs &a)
 {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= a.n) return;
     uint32_t w = a.in[i];
     f32x2 v0 = fp4x2_to_f32<0>(w), v1 = fp4x2_to_f32<1>(w), v2 = fp4x2_to_f32<2>(w), v3 = fp4x2_to_f32<3>(w);
