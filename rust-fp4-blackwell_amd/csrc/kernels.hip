@@ -35,7 +35,17 @@
     GEMV_KERNEL(SNAME, SF32, ENAME, EPI, R, 0) \
     GEMV_KERNEL(SNAME, SF32, ENAME, EPI, R, 1) \
     GEMV_KERNEL(SNAME, SF32, ENAME, EPI, R, 2)
+// K of 8193..12288 and 14337..16384 (the planner's rows per wave only)
+#define GEMV_NS_LONG(SNAME, SF32, ENAME, EPI, R) \
+    GEMV_KERNEL(SNAME, SF32, ENAME, EPI, R, 5) \
+    GEMV_KERNEL(SNAME, SF32, ENAME, EPI, R, 6) \
+    GEMV_KERNEL(SNAME, SF32, ENAME, EPI, R, 8)
 
+GEMV_NS_LONG(e8m0, 0, store, RFP4_EPI_STORE, 2)
+GEMV_NS_LONG(e8m0, 0, resid, RFP4_EPI_RESIDUAL, 1)
+GEMV_NS_LONG(e8m0, 0, resid, RFP4_EPI_RESIDUAL, 2)
+GEMV_NS_LONG(f32, 1, store, RFP4_EPI_STORE, 2)
+GEMV_NS_LONG(f32, 1, resid, RFP4_EPI_RESIDUAL, 2)
 GEMV_NS_FULL(e8m0, 0, store, RFP4_EPI_STORE, 1)
 GEMV_NS_FULL(e8m0, 0, store, RFP4_EPI_STORE, 2)
 GEMV_NS_FULL(e8m0, 0, store, RFP4_EPI_STORE, 4)

@@ -451,6 +451,8 @@ static bool gemv_has_ns(bool f32scale, int epi, int R, int ns, int W = 4)
     if (W != 4) // 8-wave workgroups: one-slice SwiGLU at R = 1, store at R = 2, residual at R = 1 of 1 or 3 slices
         return (W == 8 && ns == 1 && ((epi == RFP4_EPI_SWIGLU && R == 1) || (epi == RFP4_EPI_STORE && R == 2))) ||
                (W == 8 && !f32scale && epi == RFP4_EPI_RESIDUAL && R == 1 && (ns == 1 || ns == 3));
+    if (ns == 5 || ns == 6 || ns == 8) // long rows: store and residual, at the planner's rows per wave
+        return (epi == RFP4_EPI_STORE || epi == RFP4_EPI_RESIDUAL) && (R == 2 || (R == 1 && epi == RFP4_EPI_RESIDUAL && !f32scale));
     const bool full = ns == 0 || ns == 1 || ns == 2 || ns == 3 || ns == 4 || ns == 7;
     const bool shrt = ns == 0 || ns == 1 || ns == 2;
     if (f32scale) {
@@ -479,7 +481,9 @@ static bool gemv_has_ns(bool f32scale, int epi, int R, int ns, int W = 4)
 // heads: Llama-3.2-1B at R = 2 2683-2716 against 2774-2795 tok/s, TinyLlama's
 // 32000 rows 2270-2292 at R = 2 against 2303-2307).
 // With f32 scales (their compiled set): R = 1 for SwiGLU, R = 2 for every
-// residual GEMV, the rest as E8M0.
+// residual GEMV, the rest as E8M0.  Slice counts 5, 6 and 8 against the slice
+// loop (R = 2, us): 4096x10240 9.5 -> 6.7, 16384x10240 28.5 -> 18.3, 5120x12288
+// 18.0 -> 10.0, 4096x16384 14.3 -> 10.4; past 16384 the loop.
 GemvVariant gemv_variant(uint32_t n, uint32_t k, int epi, bool f32scale)
 {
     int ns_needed = (int)((k + 2047u) / 2048u);
