@@ -232,7 +232,8 @@ RFP4_DEV void gemv_body(const GemvArgs &a)
         // x (and norm weights) go into registers first, then every weight load
         // of this wave (NS slices x NP rows): waiting for x then never waits
         // for the weights (vmcnt retires in issue order).  A lane past the
-        // last chunk re-reads the last chunk (in bounds) and gets scale 0.
+        // last chunk re-reads the last chunk (in bounds) and keeps its sum (a
+        // zero factor would turn an infinite x of that chunk into NaN).
         constexpr int XV = NS > 0 ? (512 * NS + (int)T - 1) / (int)T : 1; // float4 of x per thread: K <= 2048 * NS
         XRegs<XV, T> xg;
         xg.issue(a.x, a.norm_w, a.k);
@@ -253,14 +254,15 @@ RFP4_DEV void gemv_body(const GemvArgs &a)
 #pragma unroll
         for (int s = 0; s < NS; s++) {
             const uint32_t c = (uint32_t)lane + 64u * (uint32_t)s;
-            const float live = c < nchunk ? 1.0f : 0.0f;
             float4 xv[8];
             const float4 *xp = (const float4 *)(xs + (size_t)min(c, clast) * GEMV_XS_CHUNK);
 #pragma unroll
             for (int j = 0; j < 8; j++) xv[j] = xp[j];
 #pragma unroll
-            for (int p = 0; p < NP; p++)
-                acc[p] = fmaf(live * scale_from_bits<SCALE_F32>(sb[s][p]), dot_chunk32(q[s][p], xv), acc[p]);
+            for (int p = 0; p < NP; p++) {
+                const float t = fmaf(scale_from_bits<SCALE_F32>(sb[s][p]), dot_chunk32(q[s][p], xv), acc[p]);
+                acc[p] = c < nchunk ? t : acc[p];
+            }
         }
     } else {
         // any K: one slice at a time

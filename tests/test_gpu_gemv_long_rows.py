@@ -28,3 +28,17 @@ def test_long_rows_equal_slice_loop(rf, stream, n, k, f32scale, resid):
         rf.check(rf.load().rfp4_debug_gemv_variant(0, -1))
     assert np.isnan(out[0][n:]).all() and np.isfinite(out[0][:n]).all()
     np.testing.assert_array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("k", [96, 2080, 8224, 10208, 14368])
+def test_infinite_last_value(rf, stream, k):
+    """An infinite x in the last, partial slice: the lanes past it, which read
+    that chunk again, add nothing (a zero factor would make the sums NaN)."""
+    n = 9
+    w = rf.DeviceBuffer.from_host(np.full(n * k // 2, 0x22, np.uint8), stream)  # every code 1.0
+    sc = rf.DeviceBuffer.from_host(np.full(n * k // 32, 127, np.uint8), stream)
+    x = np.ones(k, np.float32)
+    x[-1] = np.inf
+    y = rf.DeviceBuffer.zeroed(n, np.float32, stream)
+    rf.mx4_gemv(stream, n, k, w, sc, rf.DeviceBuffer.from_host(x, stream), y)
+    np.testing.assert_array_equal(y.to_host(n, np.float32, stream), np.full(n, np.inf, np.float32))
