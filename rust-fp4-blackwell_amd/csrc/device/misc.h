@@ -101,7 +101,11 @@ RFP4_DEV unsigned long long keys_block_max(unsigned long long best)
 RFP4_DEV void argmax_keys_body(const ArgmaxKeysArgs &a)
 {
     const unsigned long long b = keys_block_max(keys_wave_max(a.best, a.n_best));
-    if (threadIdx.x == 0) *a.out = 0xFFFFFFFFu - (uint32_t)(b & 0xFFFFFFFFull);
+    if (threadIdx.x == 0) {
+        const uint32_t tok = 0xFFFFFFFFu - (uint32_t)(b & 0xFFFFFFFFull);
+        *a.out = tok;
+        if (a.host_out) __hip_atomic_store(a.host_out, tok, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // ---------------------------------------------------------------- end of decode step

@@ -16,11 +16,15 @@
 // per thread (k is a multiple of 256 here, so rows start 16-byte aligned), a
 // workgroup per 2048 elements of a row, so that a row takes one round trip
 // (one element per thread and trip before: 700 rows x 4096 12.9 us, now 9.3).
+// The ids are in pinned host memory: one load per workgroup.
 RFP4_DEV void embed_rows_body(const RowsArgs &a)
 {
+    __shared__ uint32_t s_tok;
     const uint32_t r = blockIdx.x, i = blockIdx.y * 256u + threadIdx.x;
+    if (threadIdx.x == 0) s_tok = __hip_atomic_load(a.ids + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __syncthreads();
     if (i >= a.k / 8u) return;
-    uint32_t tok = a.ids[r];
+    uint32_t tok = s_tok;
     if (tok >= a.vocab) tok = 0;
     const u32x4 w = ((const u32x4 *)(a.embed + (size_t)tok * a.k))[i];
     const bool bf16 = a.bf16 != 0;

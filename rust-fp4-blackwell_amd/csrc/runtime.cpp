@@ -898,9 +898,9 @@ size_t mx4_gemv_argmax_workspace(uint32_t n) { return ((size_t)n + 7u) / 8u * 8u
 
 namespace rfp4 {
 
-int argmax_keys_launch(const unsigned long long *best, uint32_t n_best, uint32_t *out, hipStream_t s)
+int argmax_keys_launch(const unsigned long long *best, uint32_t n_best, uint32_t *out, uint32_t *host_out, hipStream_t s)
 {
-    ArgmaxKeysArgs ka{best, out, n_best, 0};
+    ArgmaxKeysArgs ka{best, out, host_out, n_best, 0};
     return launch("rfp4_argmax_keys", dim3(1), dim3(1024), s, &ka);
 }
 
@@ -919,7 +919,7 @@ static int gemv_argmax_launch(hipStream_t s, const char *sname, const GemvArgs &
                          mx4_gemv_argmax_workspace(args.n));
     int rc = gemv_launch_v(sname, RFP4_EPI_ARGMAX, args, s, v);
     if (rc) return rc;
-    return argmax_keys_launch((const unsigned long long *)workspace, nb, best_token, s);
+    return argmax_keys_launch((const unsigned long long *)workspace, nb, best_token, nullptr, s);
 }
 
 int mx4_gemv_argmax(rfp4_stream_t stream, uint32_t n, uint32_t k, const uint8_t *codes, const uint8_t *scales,

@@ -74,7 +74,7 @@ inline uint32_t gemv_grid(uint32_t n, const GemvVariant &v) { return (n + (uint3
 int gemv_launch_v(const char *scale_name, int epi, const GemvArgs &args, hipStream_t s, const GemvVariant &v);
 int gemv_launch(const char *scale_name, int epi, const GemvArgs &args, hipStream_t s);
 // *out = the token of the largest of an argmax GEMV's n_best keys.
-int argmax_keys_launch(const unsigned long long *best, uint32_t n_best, uint32_t *out, hipStream_t s);
+int argmax_keys_launch(const unsigned long long *best, uint32_t n_best, uint32_t *out, uint32_t *host_out, hipStream_t s);
 int attn_launch(const AttnArgs &args, int kv_f16, hipStream_t s, uint32_t max_seq_for_grid, uint32_t rows);
 // Query-head slices per KV head for an attention grid of `splits` splits
 // (args.head_split = 0 asks attn_launch for this).

@@ -67,6 +67,7 @@ typedef struct ArgmaxArgs {
 typedef struct ArgmaxKeysArgs {
     const unsigned long long *best;
     uint32_t *out;
+    uint32_t *host_out; // if non-null, the token there too (pinned host memory)
     uint32_t n_best, pad;
 } ArgmaxKeysArgs;
 
