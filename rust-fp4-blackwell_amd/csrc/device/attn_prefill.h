@@ -159,7 +159,14 @@ RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0, bool firs
     const uint32_t nk = pos0 + last_row + 1u;
     const uint32_t nblk = (nk + PF_BK - 1) / PF_BK;
     const uint32_t niter = KSP > 1 ? (nblk + KSP - 1) / KSP : nblk; // staging steps
-    const float scale = __fmul_rn(1.4426950408889634f, __fdiv_rn(1.0f, __fsqrt_rn((float)HD))); // log2(e) / sqrt(HD)
+    // The softmax scale log2(e) / sqrt(HD) in two factors: 4 times it goes into
+    // q, so that a score's exponent is a quarter of it, a power of two: score
+    // times factor minus maximum is then exact to one rounding, and 0 for the
+    // maximum itself.  (With the whole scale as the fma's factor the difference
+    // carries the rounding error of the subtracted maximum: 2^-24 of it, which
+    // for finite scores from about 2^30 on made the exponential infinite.)
+    const float qscale = 4.0f * __fmul_rn(1.4426950408889634f, __fdiv_rn(1.0f, __fsqrt_rn((float)HD)));
+    constexpr float quarter = 0.25f;
 
     // ---- Q tiles of this wave as fp16 A operands (rows past the prompt or heads past G: zero)
     f16x8 qa[MT][KS], ql[MT][KS];
@@ -175,13 +182,14 @@ RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0, bool firs
             v[0] = x0.x; v[1] = x0.y; v[2] = x0.z; v[3] = x0.w;
             v[4] = x1.x; v[5] = x1.y; v[6] = x1.z; v[7] = x1.w;
 #pragma unroll
-            for (int i = 0; i < 8; i++) v[i] = in ? v[i] : 0.0f;
+            for (int i = 0; i < 8; i++) v[i] = in ? __fmul_rn(v[i], qscale) : 0.0f;
             split_hi_lo8(v, qa[mt][k], ql[mt][k]);
         }
     }
 
     // O^T tile n: accumulator r of lane l is dimension 16 n + 4 q4 + r of row l16;
-    // the running max and sum are the lane's row's
+    // the running max (finite, also while every key so far is masked) and sum
+    // are the lane's row's
     f32x4 o[MT][NN];
     float mrun[MT], lrun[MT];
 #pragma unroll
@@ -285,7 +293,7 @@ RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0, bool firs
 #pragma unroll
                     for (int r = 0; r < 4; r++) {
                         const uint32_t key = b * PF_BK + 16u * h + 4u * q4 + (uint32_t)r;
-                        if (key > qpos) p[4 * h + r] = -3.402823466e38f;
+                        if (key > qpos) p[4 * h + r] = -INFINITY; // p is 0 whatever maximum is subtracted
                     }
             }
             // ---- online softmax (base 2) of the lane's row.  The subtracted
@@ -297,7 +305,7 @@ RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0, bool firs
             float mx = p[0];
 #pragma unroll
             for (int i = 1; i < 4 * NQ; i++) mx = fmaxf(mx, p[i]);
-            mx *= scale; // rounding is monotonic: the maximum of the scaled scores
+            mx *= quarter;
             if (__any(mx > mrun[mt] + 8.0f)) {
                 const float rowmax = xor32_max(xor16_max(mx));
                 const float mnew = rowmax > mrun[mt] + 8.0f ? rowmax : mrun[mt]; // a row's own choice, whatever its wave holds
@@ -309,7 +317,7 @@ RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0, bool firs
             }
 #pragma unroll
             for (int i = 0; i < 4 * NQ; i++) {
-                p[i] = __builtin_amdgcn_exp2f(fmaf(p[i], scale, -mrun[mt]));
+                p[i] = __builtin_amdgcn_exp2f(fmaf(p[i], quarter, -mrun[mt]));
                 lrun[mt] += p[i];
             }
             // ---- O^T += V^T P^T per 32-key chunk c (quarters 2c, 2c + 1): P^T as
