@@ -320,8 +320,9 @@ int rfp4_debug_prefill_attn(int mode);
  * attention rows, 5 the o GEMM, 6 residual add + RMSNorm + MXFP4 rows, 7 the
  * gate|up GEMM, 8 SwiGLU + MXFP4 rows, 9 the down GEMM.  -2 = no stop. */
 int rfp4_debug_prefill_stop(int after);
-/* Test hook: waves per workgroup of the matrix-core prefill attention on
- * this thread (0 = automatic, 4 or 8).  No reference counterpart. */
+/* Takes 0, 4 or 8 and has no effect: the prefill attention has one wave count
+ * per query-head group (8 waves for groups of 8, else 4 per key group).  Kept
+ * for programs built against it.  No reference counterpart. */
 int rfp4_debug_prefill_waves(int waves);
 /* Test hook (this thread): key groups per workgroup of the batched
  * prefill's attention: 0 = automatic (by grid and context length), 1 = one,
@@ -329,9 +330,9 @@ int rfp4_debug_prefill_waves(int waves);
  * blocks of the same query tiles and merge their softmax states).  No
  * reference counterpart. */
 int rfp4_debug_prefill_ksplit(int groups);
-/* Test hook: query-tile pairing of the matrix-core prefill attention on this
- * thread (0 = automatic, which is 1 now, 1 = one tile per workgroup, 2 = tiles t and
- * ntiles-1-t per workgroup).  No reference counterpart. */
+/* Takes 0, 1 or 2 and has no effect: every workgroup of the prefill attention
+ * takes one query tile.  Kept for programs built against it.  No reference
+ * counterpart. */
 int rfp4_debug_prefill_pairing(int mode);
 /* The tile and K split fp4_gemm would use for this shape (honours the test
  * hook).  No reference counterpart. */

@@ -31,7 +31,9 @@
 // one workgroup of 8 waves: 1531 rows after 517 keys 146 us, by DMA 93 us, with
 // two key groups of 4 waves 81 us, with the rarely raised maximum, uniform DMA
 // bases and two interleaved score chains 75 us (267 -> 191 us at 2048 + 2048,
-// 33 -> 20.5 us at 700 rows).  At most 128 registers keep 4 waves per SIMD.
+// 33 -> 20.5 us at 700 rows).  The kernels of 8 and 16 waves take at most 127
+// registers, which keeps 4 waves per SIMD; the one-group kernels of 4 waves,
+// planned for contexts of at most 64 keys only, take 120 to 152.
 //
 // q and p enter as hi + lo (hi = fp16(x), lo = fp16(x - hi): about 2^-22
 // relative, two MFMAs per product; K and V are fp16 already), products exact
@@ -110,7 +112,7 @@ RFP4_DEV void pf_read_v(f16x8 (&va)[4], uint32_t addr, uint32_t n0)
     }
 }
 
-// One query tile: prompt rows r0 .. r0 + BQ of KV head blockIdx.y.  QO: the
+// One query tile: prompt rows r0 .. r0 + BQ of KV head kvh.  QO: the
 // kernel variant that can quantize its output rows (AttnPrefillArgs::q_codes;
 // a separate instantiation: the epilogue's code changes how the compiler
 // schedules the main loop's LDS reads in the same function).
@@ -119,8 +121,13 @@ RFP4_DEV void pf_read_v(f16x8 (&va)[4], uint32_t addr, uint32_t n0)
 // brings KSP blocks into LDS), then merge their softmax states through LDS
 // (m the maximum, l and O rescaled by 2^(m_g - m) and summed): the serial
 // chain of blocks of a tile is KSP times shorter.
-template <int HD, int GT, int NW, bool QO, int KSP = 1>
-RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0, bool first)
+//
+// Grid (n_kv_heads, tiles): consecutive workgroups take the same query tile of
+// every KV head, the longest causal range first, so that the short ones fill
+// the end of the launch; with 8 KV heads each XCD (workgroup id % 8) keeps one
+// head's K/V in its L2.
+template <int HD, int GT, int NW, bool QO = false, int KSP = 1>
+RFP4_DEV void attn_prefill_body(const AttnPrefillArgs &a)
 {
     const uint32_t pos0 = a.pos0, nrows = a.rows;
     constexpr int BQ = attn_prefill_rows(GT, NW);    // prompt rows per workgroup
@@ -145,13 +152,13 @@ RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0, bool firs
     __shared__ __attribute__((aligned(1024))) uint8_t lds_raw[NST * STAGE];
     pf_lds_u8 *lds = (pf_lds_u8 *)lds_raw;
 
-    const uint32_t kvh = blockIdx.x % a.n_kv_heads;
+    const uint32_t kvh = blockIdx.x, r0 = (a.tile - blockIdx.y) * BQ;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     // key group; wave within it (KSP = 1: the plain kernel's code, group 0)
     const int kgrp = KSP > 1 ? wid / NW : 0, wave = KSP > 1 ? wid % NW : wid;
     const uint32_t l16 = (uint32_t)lane & 15u, q4 = (uint32_t)lane >> 4;
-    const uint32_t G = a.n_heads / a.n_kv_heads;
+    const uint32_t G = a.group;
     const uint16_t *kc = a.kc + (size_t)kvh * a.hs;
     const uint16_t *vc = a.vc + (size_t)kvh * a.hs;
     // keys of this workgroup: 0 .. position of its last row
@@ -245,7 +252,6 @@ RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0, bool firs
     const uint32_t kaddr = lds0 + l16 * RB + ((q4 ^ pf_kswz<HD>(l16)) << 4);
     const uint32_t vrow = 4u * q4 + (l16 >> 2);
     const uint32_t vaddr = lds0 + PF_BK * RB + vrow * RB + ((((l16 & 3u) >> 1) ^ pf_vswz<HD>(vrow)) << 4) + 8u * (l16 & 1u);
-    if (!first) __syncthreads(); // the previous tile's LDS reads are done
 #pragma unroll
     for (uint32_t i = 0; i + 1u < NST; i++) stage_dma(i, i);
 
@@ -458,22 +464,4 @@ RFP4_DEV void attn_prefill_tile(const AttnPrefillArgs &a, uint32_t r0, bool firs
             }
         }
     }
-}
-
-// Grid (one dimension, n_kv_heads x tiles): consecutive workgroups take the same query tile
-// of every KV head, the longest causal range first, so that the short
-// ones fill the end of the launch; with 8 KV heads each XCD (workgroup id % 8)
-// keeps one head's K/V in its L2.
-// Workgroup y of a head: query tile ntiles - 1 - y, or, paired, tiles ntiles
-// - 1 - y and y, so that every workgroup walks ntiles + 1 key ranges' worth of
-// blocks.
-template <int HD, int GT, int NW = 4, bool QO = false, int KSP = 1>
-RFP4_DEV void attn_prefill_body(const AttnPrefillArgs &a)
-{
-    constexpr uint32_t BQ = (uint32_t)attn_prefill_rows(GT, NW);
-    const uint32_t ntiles = (a.rows + BQ - 1u) / BQ, y = blockIdx.x / a.n_kv_heads, t0 = ntiles - 1u - y;
-    const uint32_t npass = a.paired && y < t0 ? 2u : 1u;
-#pragma nounroll
-    for (uint32_t pass = 0; pass < npass; pass++)
-        attn_prefill_tile<HD, GT, NW, QO, KSP>(a, (pass == 0 ? t0 : y) * BQ, pass == 0);
 }

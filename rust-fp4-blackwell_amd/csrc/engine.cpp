@@ -522,7 +522,7 @@ static int enqueue_prefill(llama_engine *e, uint32_t n, uint32_t pos0)
             // hook wants the f32 rows
             attn_q = stop != (int)(10u * l + 3u) && prefill_attn_quant_mode() == 0;
             AttnPrefillArgs pa{e->pf_c, kc, vc, attn_q ? nullptr : e->pf_a, hd, (uint64_t)e->max_seq_alloc * hd, nqkv, qd,
-                               c.n_heads, c.n_kv_heads, pos0, n, 0u}; // pairing: chosen by the launcher
+                               c.n_heads, c.n_kv_heads, pos0, n, 0u, 0u, nullptr, nullptr, nullptr};
             if (attn_q) {
                 pa.q_codes = e->pf_codes;
                 pa.q_scales = e->pf_scales;

@@ -121,18 +121,10 @@ ATTN_KERNELS(128, f16, uint16_t)
     K256 void rfp4_attn_prefill_hd##HD##_g1_w4(AttnPrefillArgs a) { attn_prefill_body<HD, 1, 4>(a); } \
     K256 void rfp4_attn_prefill_hd##HD##_g2_w4(AttnPrefillArgs a) { attn_prefill_body<HD, 2, 4>(a); } \
     K256 void rfp4_attn_prefill_hd##HD##_g4_w4(AttnPrefillArgs a) { attn_prefill_body<HD, 4, 4>(a); } \
-    K256 void rfp4_attn_prefill_hd##HD##_g8_w4(AttnPrefillArgs a) { attn_prefill_body<HD, 8, 4>(a); } \
-    K512Q void rfp4_attn_prefill_hd##HD##_g1_w8(AttnPrefillArgs a) { attn_prefill_body<HD, 1, 8>(a); } \
-    K512Q void rfp4_attn_prefill_hd##HD##_g2_w8(AttnPrefillArgs a) { attn_prefill_body<HD, 2, 8>(a); } \
-    K512Q void rfp4_attn_prefill_hd##HD##_g4_w8(AttnPrefillArgs a) { attn_prefill_body<HD, 4, 8>(a); } \
     K512Q void rfp4_attn_prefill_hd##HD##_g8_w8(AttnPrefillArgs a) { attn_prefill_body<HD, 8, 8>(a); } \
     K256 void rfp4_attn_prefill_hd##HD##_g1_w4_q(AttnPrefillArgs a) { attn_prefill_body<HD, 1, 4, true>(a); } \
     K256 void rfp4_attn_prefill_hd##HD##_g2_w4_q(AttnPrefillArgs a) { attn_prefill_body<HD, 2, 4, true>(a); } \
     K256 void rfp4_attn_prefill_hd##HD##_g4_w4_q(AttnPrefillArgs a) { attn_prefill_body<HD, 4, 4, true>(a); } \
-    K256 void rfp4_attn_prefill_hd##HD##_g8_w4_q(AttnPrefillArgs a) { attn_prefill_body<HD, 8, 4, true>(a); } \
-    K512Q void rfp4_attn_prefill_hd##HD##_g1_w8_q(AttnPrefillArgs a) { attn_prefill_body<HD, 1, 8, true>(a); } \
-    K512Q void rfp4_attn_prefill_hd##HD##_g2_w8_q(AttnPrefillArgs a) { attn_prefill_body<HD, 2, 8, true>(a); } \
-    K512Q void rfp4_attn_prefill_hd##HD##_g4_w8_q(AttnPrefillArgs a) { attn_prefill_body<HD, 4, 8, true>(a); } \
     K512Q void rfp4_attn_prefill_hd##HD##_g8_w8_q(AttnPrefillArgs a) { attn_prefill_body<HD, 8, 8, true>(a); }
 ATTN_PREFILL_KERNELS(64)
 ATTN_PREFILL_KERNELS(128)

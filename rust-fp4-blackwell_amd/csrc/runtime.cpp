@@ -518,9 +518,7 @@ static thread_local int t_qkva = 0; // engines created on this thread: 0 fused q
 int qkva_mode() { return t_qkva; }
 
 static thread_local int t_prefill_attn = 0; // 0 matrix-core prefill kernel, 1 one decode-kernel row per prompt row
-static thread_local int t_prefill_waves = 0; // prefill attention waves per workgroup (0 = automatic)
-static thread_local int t_prefill_pairing = 0; // 0 automatic, 1 one query tile per workgroup, 2 paired tiles
-static thread_local int t_prefill_ksplit = 0; // prefill attention key groups per workgroup (0 automatic, 1, 2)
+static thread_local int t_prefill_ksplit = 0; // prefill attention key groups per workgroup (0 automatic, 1, 2 or 4)
 int prefill_attn_mode() { return t_prefill_attn; }
 static thread_local int t_prefill_stop = -2; // stage after which the batched prefill stops (-2: none)
 int prefill_stop() { return t_prefill_stop; }
@@ -621,8 +619,7 @@ extern "C" int rfp4_debug_prefill_waves(int waves)
 {
     using namespace rfp4;
     if (waves != 0 && waves != 4 && waves != 8) return set_error(RFP4_E_INVALID, "prefill attention waves must be 0 (auto), 4 or 8");
-    t_prefill_waves = waves;
-    return RFP4_OK;
+    return RFP4_OK; // one wave count is compiled per query-head group
 }
 
 extern "C" int rfp4_debug_prefill_ksplit(int groups)
@@ -638,8 +635,7 @@ extern "C" int rfp4_debug_prefill_pairing(int mode)
 {
     using namespace rfp4;
     if (mode < 0 || mode > 2) return set_error(RFP4_E_INVALID, "pairing mode must be 0 (auto), 1 (off) or 2 (on)");
-    t_prefill_pairing = mode;
-    return RFP4_OK;
+    return RFP4_OK; // every workgroup takes one query tile
 }
 
 extern "C" int rfp4_debug_prefill_stop(int after)
@@ -762,8 +758,7 @@ int attn_prefill_launch(const AttnPrefillArgs &a, uint32_t head_dim, hipStream_t
     const uint32_t g = attn_group_pad(a.n_heads / a.n_kv_heads);
     // 4 waves (16 prompt rows of 4 heads, one 16-row tile per wave) per key
     // group, 8 where the KV head has 8 query heads.
-    uint32_t waves = g == 8u ? 8u : 4u;
-    if (t_prefill_waves) waves = (uint32_t)t_prefill_waves;
+    const uint32_t waves = g == 8u ? 8u : 4u;
     const uint32_t bq = (uint32_t)attn_prefill_rows((int)g, (int)waves); // prompt rows per workgroup
     const uint32_t ntiles = (a.rows + bq - 1) / bq;
     const uint64_t keys = (uint64_t)a.pos0 + a.rows, wgs = (uint64_t)ntiles * a.n_kv_heads;
@@ -779,25 +774,21 @@ int attn_prefill_launch(const AttnPrefillArgs &a, uint32_t head_dim, hipStream_t
     // where a workgroup per CU holds the grid (16 waves fill a CU), else two,
     // and one for contexts of a few blocks.
     const uint64_t cus = g_rt ? (uint64_t)g_rt->num_cus : 256u;
-    uint32_t ks = waves == 8u ? (g == 8u && keys > 512u ? 2u : 1u) : g == 8u || keys <= 64u ? 1u : keys > 1024u && wgs <= cus ? 4u : 2u;
-    if (t_prefill_ksplit) {
-        ks = (uint32_t)t_prefill_ksplit;
-        if (ks == 4u && !(waves == 4u && g < 8u)) ks = 2u;
-        if (ks == 2u && !((waves == 4u && g < 8u) || (waves == 8u && g == 8u))) ks = 1u;
-    }
-    // Pairing tile t with ntiles - 1 - t in one workgroup evens out the causal
-    // ranges of a grid of one workgroup per CU; no longer chosen (two
-    // workgroups per CU, the longest first, are as fast or faster: 2048 rows of
-    // 8B heads 76.6 against 82.6 us paired).
-    const bool paired = t_prefill_pairing == 2;
+    uint32_t ks = g == 8u ? (keys > 512u ? 2u : 1u) : keys <= 64u ? 1u : keys > 1024u && wgs <= cus ? 4u : 2u;
+    if (t_prefill_ksplit) ks = std::min((uint32_t)t_prefill_ksplit, g == 8u ? 2u : 4u);
     char name[48];
     char sfx[8] = "";
     if (ks > 1u) snprintf(sfx, sizeof sfx, "_s%u", ks);
     snprintf(name, sizeof name, "rfp4_attn_prefill_hd%u_g%u_w%u%s%s", head_dim, g, waves, a.q_codes ? "_q" : "", sfx);
     AttnPrefillArgs args = a;
-    args.paired = paired ? 1u : 0u;
-    const uint32_t gx = paired ? (ntiles + 1) / 2 : ntiles;
-    return launch(name, dim3(a.n_kv_heads * gx), dim3(64u * waves * ks), s, &args);
+    args.group = a.n_heads / a.n_kv_heads;
+    for (uint32_t left = ntiles; left;) { // a grid's second dimension takes at most 65535 tiles
+        const uint32_t n = std::min(left, 65535u);
+        args.tile = left - 1u;
+        if (int rc = launch(name, dim3(a.n_kv_heads, n), dim3(64u * waves * ks), s, &args)) return rc;
+        left -= n;
+    }
+    return RFP4_OK;
 }
 
 uint32_t attn_group_pad(uint32_t group) { return group <= 1u ? 1u : group <= 2u ? 2u : group <= 4u ? 4u : 8u; }
@@ -1082,7 +1073,8 @@ int attn_prefill_f16(rfp4_stream_t stream, uint32_t n_heads, uint32_t n_kv_heads
         return set_error(RFP4_E_SHAPE, "attn_prefill_f16: q row stride %u < %u", q_row_stride, n_heads * head_dim);
     if (rows && out_row_stride < n_heads * head_dim)
         return set_error(RFP4_E_SHAPE, "attn_prefill_f16: out row stride %u < %u", out_row_stride, n_heads * head_dim);
-    AttnPrefillArgs a{q, kc, vc, out, token_stride, head_stride, q_row_stride, out_row_stride, n_heads, n_kv_heads, pos0, rows, 0u};
+    AttnPrefillArgs a{q, kc, vc, out, token_stride, head_stride, q_row_stride, out_row_stride, n_heads, n_kv_heads, pos0, rows, 0u, 0u,
+                      nullptr, nullptr, nullptr};
     return attn_prefill_launch(a, head_dim, (hipStream_t)stream);
 }
 

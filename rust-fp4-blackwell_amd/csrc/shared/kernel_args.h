@@ -136,7 +136,7 @@ typedef struct AttnPrefillArgs {
     float *out;              // row r: out + r*out_rs, [n_heads][head_dim]
     uint64_t ts, hs;
     uint32_t q_rs, out_rs, n_heads, n_kv_heads, pos0, rows;
-    uint32_t paired;         // nonzero: workgroup x takes query tiles ntiles-1-x and x (grid ceil(ntiles/2))
+    uint32_t group, tile;    // query heads per KV head; the first workgroups' query tile (attn_prefill_launch fills both in)
     // Optional (null = off): the output rows quantized to MXFP4 per 32 as the
     // row quantizer does it, codes [rows][n_heads*head_dim/2], scales
     // [rows][n_heads*head_dim/32] and, if not null, their step-blocked copy
