@@ -253,7 +253,8 @@ RFP4_DEV void attn_prefill_body(const AttnPrefillArgs &a)
     const uint32_t vrow = 4u * q4 + (l16 >> 2);
     const uint32_t vaddr = lds0 + PF_BK * RB + vrow * RB + ((((l16 & 3u) >> 1) ^ pf_vswz<HD>(vrow)) << 4) + 8u * (l16 & 1u);
 #pragma unroll
-    for (uint32_t i = 0; i + 1u < NST; i++) stage_dma(i, i);
+    for (uint32_t i = 0; i + 1u < NST; i++)
+        if (KSP > 1 || i < niter) stage_dma(i, i);
 
     // the block's scores, softmax and P V from the stage at byte sb (this key
     // group's block b of the step in slot kgrp; none past the last block)
@@ -349,22 +350,29 @@ RFP4_DEV void attn_prefill_body(const AttnPrefillArgs &a)
     // Step i: wait for this wave's DMAs of step i (those of the NST - 2 steps
     // behind it may be in flight), then the barrier: every wave's copies of
     // step i are in LDS and every wave is past its reads of step i - 1, whose
-    // buffer the DMAs of step i + NST - 1 then overwrite.
+    // buffer the DMAs of step i + NST - 1 then overwrite.  With one key group
+    // (contexts of a few blocks) no DMA is issued past the last block, and the
+    // last step waits for all: the copies that nothing reads were 0.2 to 0.3
+    // of the 5.6 us of 51 rows of TinyLlama's heads.  With more groups the
+    // branch around the DMAs costs more than the copies (100 rows after 4000
+    // keys of the 8B heads 55.9 us without it, 58.2 with).
     uint32_t buf = 0;
     for (uint32_t it = 0; it < niter; it++) {
-        __builtin_amdgcn_s_waitcnt(PF_VMCNT(NI * (NST - 2u)));
+        if (KSP > 1 || it + 1u < niter) __builtin_amdgcn_s_waitcnt(PF_VMCNT(NI * (NST - 2u)));
+        else __builtin_amdgcn_s_waitcnt(PF_VMCNT(0));
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        stage_dma(it + NST - 1u, buf == 0u ? NST - 1u : buf - 1u);
+        if (KSP > 1 || it + NST - 1u < niter) stage_dma(it + NST - 1u, buf == 0u ? NST - 1u : buf - 1u);
         block(it * KSP + (uint32_t)kgrp, buf * STAGE);
         buf = buf + 1u == NST ? 0u : buf + 1u;
     }
-    // the last DMAs (past the end) land before the LDS is used again
-    __builtin_amdgcn_s_waitcnt(PF_VMCNT(0));
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    if (KSP > 1) { // the last DMAs (past the end) land before the merge uses the LDS again
+        __builtin_amdgcn_s_waitcnt(PF_VMCNT(0));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    }
 
     // the row's sum over its four lanes
 #pragma unroll
