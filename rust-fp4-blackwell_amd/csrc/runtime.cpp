@@ -1067,6 +1067,9 @@ int attn_prefill_f16(rfp4_stream_t stream, uint32_t n_heads, uint32_t n_kv_heads
     if (!runtime()) return set_error(RFP4_E_NOT_INIT, "rfp4_init has not been called");
     if (((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) & 15u || q_row_stride % 4u || (token_stride * 2u) % 16u)
         return set_error(RFP4_E_ALIGN, "attn_prefill_f16: q rows and K/V rows must start 16-byte aligned");
+    if (rows && n_kv_heads > 1 && (head_stride * 2u) % 16u) // 16-byte copies into LDS from every head's rows
+        return set_error(RFP4_E_ALIGN, "attn_prefill_f16: K/V rows must start 16-byte aligned (head stride %llu)",
+                         (unsigned long long)head_stride);
     if ((uintptr_t)out & 15u || out_row_stride % 4u)
         return set_error(RFP4_E_ALIGN, "attn_prefill_f16: out rows must start 16-byte aligned");
     if (rows && q_row_stride < n_heads * head_dim)
