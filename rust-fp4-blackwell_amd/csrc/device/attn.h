@@ -811,12 +811,14 @@ struct AttnSplit {
         }
         __syncthreads();
 
-        // The output loops step by blockDim.x (always 256 here): with the constant
-        // the same kernels are slower, unrolled or not (16 TinyLlama steps at
-        // context 200: 6941 us with it, 6908 without).
+        // The output loops' step is 256; the fused kernel is faster with it read
+        // from the launch, unrolled or not (16 TinyLlama steps at context 200: 6908
+        // us, 6941 with the constant), the stand-alone ones by 1-2 % with the
+        // constant (f32, 32 heads over 8, 200 keys: 4.40 us, 4.49 read).
+        const uint32_t step = QT ? blockDim.x : 256u;
         if (nsplit == 1) {
             // one split holds the whole sequence: normalise and write the heads' outputs
-            for (uint32_t i = tid; i < G * HD; i += blockDim.x) {
+            for (uint32_t i = tid; i < G * HD; i += step) {
                 const uint32_t g = i / HD, d = i % HD;
                 const float v = vred[0][g][d] + vred[1][g][d] + vred[2][g][d] + vred[3][g][d];
                 const float l = (s_lred[0][g] + s_lred[1][g]) + (s_lred[2][g] + s_lred[3][g]);
@@ -832,7 +834,7 @@ struct AttnSplit {
         const uint32_t stride = HD + 4;
         if (TAG) {
             const uint32_t tag = seq;
-            for (uint32_t i = tid; i < G * HD; i += blockDim.x) {
+            for (uint32_t i = tid; i < G * HD; i += step) {
                 const uint32_t g = i / HD, d = i % HD;
                 const float v = vred[0][g][d] + vred[1][g][d] + vred[2][g][d] + vred[3][g][d];
                 const float l = (s_lred[0][g] + s_lred[1][g]) + (s_lred[2][g] + s_lred[3][g]);
@@ -849,7 +851,7 @@ struct AttnSplit {
             return;
         }
         const bool inmerge = a.counters != nullptr;
-        for (uint32_t i = tid; i < G * HD; i += blockDim.x) {
+        for (uint32_t i = tid; i < G * HD; i += step) {
             uint32_t g = i / HD, d = i % HD;
             float v = vred[0][g][d] + vred[1][g][d] + vred[2][g][d] + vred[3][g][d];
             size_t base = ((size_t)(hbase + g) * a.max_splits + split) * stride;
