@@ -340,6 +340,13 @@ int rfp4_gemm_plan(uint32_t m, uint32_t n, uint32_t k, int *tile_m, int *tile_n,
 /* The kernel fp4_gemm would launch for this shape, with its K split
  * ("<kernel>/kz<splits>"; the few-row kernel's name carries its plan). */
 int rfp4_gemm_plan_kernel(uint32_t m, uint32_t n, uint32_t k, char *buf, size_t cap);
+/* The kernel that the batched prefill runs for a projection of m rows where it
+ * has a fused epilogue, "" where the plain GEMM and a row kernel do the work:
+ * with head_dim = 0 the gate|up projection of n = ffn pairs (SwiGLU and MXFP4
+ * rows), else the q|k|v projection of n columns (RoPE and K/V rows).  Planned
+ * apart from fp4_gemm; honours the test hooks but those that turn an epilogue
+ * off.  No reference counterpart. */
+int rfp4_prefill_epilogue_kernel(uint32_t m, uint32_t n, uint32_t k, uint32_t head_dim, char *buf, size_t cap);
 
 /* ------------------------------------------------------------------ test hooks
  * Raw single-tile MFMA (layout pinning, the role of trackb/fp4_mapping_test.cu

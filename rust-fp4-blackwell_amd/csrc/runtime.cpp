@@ -1736,6 +1736,19 @@ int rfp4_gemm_plan_kernel(uint32_t m, uint32_t n, uint32_t k, char *buf, size_t 
     return RFP4_OK;
 }
 
+int rfp4_prefill_epilogue_kernel(uint32_t m, uint32_t n, uint32_t k, uint32_t head_dim, char *buf, size_t cap)
+{
+    if (!g_rt) return set_error(RFP4_E_NOT_INIT, "rfp4_init has not been called");
+    if (!buf || cap == 0) return set_error(RFP4_E_INVALID, "prefill_epilogue_kernel: null buffer");
+    uint32_t cols = 0;
+    RopeKernel rk{};
+    const char *name = head_dim ? (gemm_rope_ok(m, n, k, head_dim) && gemm_rope_kernel(m, n, k, rk) ? rk.name : nullptr)
+                                : gemm_swiglu_kernel(m, n, k, cols);
+    if (!name) name = "";
+    if (strlen(name) + 1 > cap) return set_error(RFP4_E_CAPACITY, "prefill_epilogue_kernel: %zu bytes needed", strlen(name) + 1);
+    memcpy(buf, name, strlen(name) + 1);
+    return RFP4_OK;
+}
 
 int rfp4_mma_tile16(rfp4_stream_t stream, const uint32_t *a, const uint32_t *b, const uint32_t *sa,
                     const uint32_t *sb, float *out)

@@ -109,6 +109,7 @@ _SIGS = {
     "rfp4_debug_attn_chunk": (I32, [U32]),
     "rfp4_gemm_plan": (I32, [U32, U32, U32, P, P, P]),
     "rfp4_gemm_plan_kernel": (I32, [U32, U32, U32, C.c_char_p, SZ]),
+    "rfp4_prefill_epilogue_kernel": (I32, [U32, U32, U32, U32, C.c_char_p, SZ]),
     "rfp4_mma_tile16": (I32, [P, P, P, P, P, P]),
     "rfp4_mma_tile32": (I32, [P, P, P, P, P, P]),
     "rfp4_selftest_cvt_fp4": (I32, [P, U32, P, P]),
@@ -510,6 +511,14 @@ def gemm_plan_kernel(m, n, k) -> str:
     """The kernel (and K split) fp4_gemm launches for this shape."""
     buf = C.create_string_buffer(96)
     check(load().rfp4_gemm_plan_kernel(m, n, k, buf, 96))
+    return buf.value.decode()
+
+
+def prefill_epilogue_kernel(m, n, k, head_dim=0) -> str:
+    """The kernel of the prefill's gate|up (n = ffn) or, with a head_dim, q|k|v
+    projection with its fused epilogue; empty where a row kernel does that work."""
+    buf = C.create_string_buffer(96)
+    check(load().rfp4_prefill_epilogue_kernel(m, n, k, head_dim, buf, 96))
     return buf.value.decode()
 
 

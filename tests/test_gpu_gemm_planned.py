@@ -37,3 +37,11 @@ def test_planned_gemm(rf, stream, m, n, k):
     got = out.to_host(m * n, np.float32, stream).reshape(m, n)
     bad = abs(got - a @ w.T) > 1e-5 * (abs(a) @ abs(w).T)
     assert not bad.any(), (rf.gemm_plan_kernel(m, n, k), int(bad.sum()))
+
+
+def test_prefill_epilogue_planned(rf, stream):
+    """The projections whose plan has a fused epilogue, by kind."""
+    assert rf.prefill_epilogue_kernel(700, 14336, 4096) == "rfp4_gemm_256x256_ppsw"
+    assert rf.prefill_epilogue_kernel(128, 5632, 2048).endswith("_sw")
+    assert rf.prefill_epilogue_kernel(700, 6144, 4096, 128).endswith("_rope")
+    assert rf.prefill_epilogue_kernel(700, 6144, 4096, 96) == ""

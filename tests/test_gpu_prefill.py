@@ -204,18 +204,18 @@ def test_engine_step_blocked_weight_scales(rf):
 
 def test_prefill_swiglu_in_gemm_epilogue(rf, orc):
     """Llama-3-8B widths, 450 prompt rows (the second 256-row tile ragged):
-    the gate|up GEMM's plan is the 256x256 ping-pong tile, so SwiGLU and the
-    MXFP4 rows of its output come from the GEMM's epilogue.  Every stage on
+    the gate|up projection is planned as the 256x256 ping-pong kernel whose
+    epilogue makes SwiGLU and the MXFP4 rows of its output.  Every stage on
     identical inputs within its bar (the SwiGLU rows against the exact values
     of the plain GEMM's output, which the stage hook stopped after the GEMM
     still writes), and against the GEMM + row kernel path (rfp4_debug_prefill_
     swiglu(1)): the same scale bytes and codes but where the two f32 sums lie
     at a rounding boundary (their K orders differ), and the same next token."""
     cfg, seed, n = W8B, 0x5A1F, 450
-    assert rf.gemm_plan_kernel(n, 2 * cfg["ffn"], cfg["dim"]).startswith("rfp4_gemm_256x256_pp/kz1")
     prompt = np.random.default_rng(450).integers(0, cfg["vocab"], n, dtype=np.uint32)
     print("prefill at 8B widths, 450 rows, SwiGLU in the gate|up epilogue", flush=True)
     eng = _engine(rf, cfg, seed)
+    assert rf.prefill_epilogue_kernel(n, cfg["ffn"], cfg["dim"]) == "rfp4_gemm_256x256_ppsw"
     ref = orc.Model(cfg, seed)
     tok = check_prefill_stages(rf, orc, eng, ref, cfg, prompt, 0)
     ffn = cfg["ffn"]
@@ -274,6 +274,7 @@ def test_prefill_rope_in_gemm_epilogue(rf, orc, cfg, n, pos0, tile, nst, plan):
         rf.debug_gemm_plan(tile, 1)
         rf.check(lib.rfp4_debug_gemm_stages(nst))
         assert rf.gemm_plan_kernel(n, nqkv, dim) == plan
+        assert rf.prefill_epilogue_kernel(n, nqkv, dim, hd) == plan.split("/")[0] + "_rope"
         if pos0:
             assert eng.prefill(head, 0) == ref.prefill(head, 0)
         tok = check_prefill_stages(rf, orc, eng, ref, cfg, prompt, pos0)
@@ -395,6 +396,7 @@ def test_prefill_swiglu_epilogue_128x128(rf, orc, cfg, n, nst, kernel):
         rf.debug_gemm_plan(2, 1)
         rf.check(lib.rfp4_debug_gemm_stages(nst))
         assert rf.gemm_plan_kernel(n, 2 * ffn, cfg["dim"]) == kernel
+        assert rf.prefill_epilogue_kernel(n, ffn, cfg["dim"]) == kernel.split("/")[0] + "_sw"
         tok = check_prefill_stages(rf, orc, eng, ref, cfg, prompt, 0)
         for mode in (0, 1):
             rf.check(lib.rfp4_debug_prefill_swiglu(mode))
