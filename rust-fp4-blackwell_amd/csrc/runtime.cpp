@@ -1406,11 +1406,12 @@ GemmPlan gemm_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t num_cus, GemmKin
     return p;
 }
 
+// The estimate of a tiled kernel's plan.
 float gemm_plan_cost(const GemmPlan &p, uint32_t m, uint32_t n, uint32_t k, uint32_t cus)
 {
     for (const GemmCost &c : kGemmCost)
         if (c.tile == p.tile && c.nst == p.nst) return gemm_cost(c, p.kz, m, n, k, cus);
-    return 0.0f; // the few-row kernel
+    return INFINITY; // not a compiled kernel
 }
 
 // The 8-wave ping-pong kernel (rfp4_gemm_<tile>_pp) for a plan of the
@@ -1547,7 +1548,11 @@ int gemm_launch(hipStream_t stream, uint32_t m, uint32_t n, uint32_t k, const ui
 // (64-column pairs).  Null: none, or the plain GEMM's best plan and the row
 // kernel (about 3 us and the f32 gate|up rows there and back) take less:
 // measured so at 48 rows of TinyLlama (10.6 us against 11.6), not from 128 rows
-// on (11.0 against 12.2; Llama-3-8B at 200 rows 30.4 against 35.5).
+// on (11.0 against 12.2; Llama-3-8B at 200 rows 30.4 against 35.5).  The
+// few-row kernel, planned only for narrow matrices, has no estimate and needs
+// none: with the row kernel's 3 us it is always ahead (8192x2048 at 32 rows 5.6
+// us against 9.9 for 128x128, 8192x4096 8.0 / 14.6, 4096x2048 at 64 rows 5.3 /
+// 10.2, 4096x1024 4.5 / 7.8).
 static const char *gemm_swiglu_kernel(uint32_t m, uint32_t ffn, uint32_t k, uint32_t &cols)
 {
     Runtime *rt = g_rt;
@@ -1558,6 +1563,7 @@ static const char *gemm_swiglu_kernel(uint32_t m, uint32_t ffn, uint32_t k, uint
     const bool pp = gemm_use_pp(p, m, 2u * ffn, k);
     if (t_gemm_tile < 0 && !t_gemm_stages) {
         const GemmPlan plain = gemm_plan(m, 2u * ffn, k, cus, GEMM_LAYER);
+        if (plain.tile == kGemmSkinny) return nullptr;
         const float rows = 3.0f + (float)m * (float)ffn * (16.0f / 4.0e6f);
         if (gemm_plan_cost(p, m, 2u * ffn, k, cus) > gemm_plan_cost(plain, m, 2u * ffn, k, cus) + rows) return nullptr;
     }

@@ -40,7 +40,11 @@ def test_planned_gemm(rf, stream, m, n, k):
 
 
 def test_prefill_epilogue_planned(rf, stream):
-    """The projections whose plan has a fused epilogue, by kind."""
+    """Where the plain gate|up GEMM is the few-row kernel (narrow matrices to 64
+    rows) there is no SwiGLU epilogue; wide or tall ones have it."""
+    assert rf.gemm_plan_kernel(64, 4096, 2048).startswith("rfp4_gemm_rows_")
+    for m, ffn, k in ((32, 4096, 2048), (64, 2048, 2048), (64, 2048, 1024)):
+        assert rf.prefill_epilogue_kernel(m, ffn, k) == ""
     assert rf.prefill_epilogue_kernel(700, 14336, 4096) == "rfp4_gemm_256x256_ppsw"
     assert rf.prefill_epilogue_kernel(128, 5632, 2048).endswith("_sw")
     assert rf.prefill_epilogue_kernel(700, 6144, 4096, 128).endswith("_rope")
