@@ -33,7 +33,7 @@
 // bases and two interleaved score chains 75 us (267 -> 191 us at 2048 + 2048,
 // 33 -> 20.5 us at 700 rows).  The kernels of 8 and 16 waves take at most 127
 // registers, which keeps 4 waves per SIMD; the one-group kernels of 4 waves,
-// planned for contexts of at most 64 keys only, take 120 to 152.
+// planned for contexts of two key blocks only, take 120 to 152.
 //
 // q and p enter as hi + lo (hi = fp16(x), lo = fp16(x - hi): about 2^-22
 // relative, two MFMAs per product; K and V are fp16 already), products exact

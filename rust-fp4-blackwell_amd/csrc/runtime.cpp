@@ -765,16 +765,21 @@ int attn_prefill_launch(const AttnPrefillArgs &a, uint32_t head_dim, hipStream_t
     // Key groups per workgroup (alternate key blocks, the states merged at the
     // end): a tile's serial chain of blocks halves or quarters, for a merge of
     // 1-3 us.  Measured (us, 1 / 2 / 4 groups of 4 waves): Llama-3-8B heads, 64
-    // rows 7.1 / 7.3 / 9.9, 512 rows 19.6 / 15.3 / 16.8, 2048 rows 83.7 / 76.6 /
-    // 91.9, 100 rows after 4000 keys 108 / 63.5 / 56.1; 8 heads of one group
-    // each, 1024 rows 31.9 / 22.0 / 21.8, 2048 rows 59.7 / 38.9 / 35.7.  Two
-    // groups of 8 waves (8 query heads per KV head; 1 / 2 groups): TinyLlama
-    // heads, 333 rows 10.6 / 11.2, 700 rows 17.0 / 16.9, 2048 rows 49.6 / 44.1;
-    // 100 rows after 4000 keys 69.2 / 59.5.  So: four groups for long chains
-    // where a workgroup per CU holds the grid (16 waves fill a CU), else two,
-    // and one for contexts of a few blocks.
+    // rows 5.8 / 6.9 / 9.5, 65 rows 7.9 / 7.2 / 9.9, 512 rows 19.0 / 14.8 / 15.7,
+    // 2048 rows 79.0 / 76.0 / 89.2, 100 rows after 4000 keys 113 / 68.1 / 56.2; 8
+    // single heads of 128, 1024 rows 32.2 / 21.8 / 20.9, 2048 rows 60.2 / 37.6 /
+    // 33.3; 32 heads of 64 over 8, 84 rows after 26 keys 5.2 / 5.5 / 6.9, 128 rows
+    // 5.1 / 5.5 / 7.0, 129 rows 6.5 / 6.0 / 7.1.  Two groups of 8 waves (8 query
+    // heads per KV head; 1 / 2 groups): TinyLlama heads, 333 rows 10.4 / 10.9, 512
+    // rows 13.1 / 13.2, 700 rows 16.7 / 16.3, 2048 rows 48.2 / 43.6; 100 rows after
+    // 4000 keys 73.0 / 60.9.  So: four groups for long chains where a workgroup
+    // per CU holds the grid (16 waves fill a CU), else two, and one up to two key
+    // blocks (of 64 keys at head dim 64, 32 at 128).
     const uint64_t cus = g_rt ? (uint64_t)g_rt->num_cus : 256u;
-    uint32_t ks = g == 8u ? (keys > 512u ? 2u : 1u) : keys <= 64u ? 1u : keys > 1024u && wgs <= cus ? 4u : 2u;
+    uint32_t ks = g == 8u ? (keys > 512u ? 2u : 1u)
+                  : keys <= (head_dim == 64u ? 128u : 64u) ? 1u
+                  : keys > 1024u && wgs <= cus             ? 4u
+                                                           : 2u;
     if (t_prefill_ksplit) ks = std::min((uint32_t)t_prefill_ksplit, g == 8u ? 2u : 4u);
     char name[48];
     char sfx[8] = "";

@@ -34,8 +34,9 @@ def test_key_groups(rf, orc, stream, nh, nkv, hd, pos0, rows):
     _run(rf, orc, stream, nh, nkv, hd, pos0, rows, ksplit=2 if nh // nkv == 8 else 4)
 
 
-# the planner's own choice on both sides of its lines (64, 512 and 1024 keys)
-@pytest.mark.parametrize("nh,nkv,hd,pos0,rows", [(4, 1, 64, 0, 64), (4, 1, 64, 0, 65), (8, 1, 64, 500, 12), (8, 1, 128, 500, 13),
+# the planner's own choice on both sides of its lines (64, 128, 512 and 1024 keys)
+@pytest.mark.parametrize("nh,nkv,hd,pos0,rows", [(4, 1, 64, 0, 64), (4, 1, 64, 0, 65), (4, 1, 64, 0, 128), (2, 1, 64, 100, 29),
+                                                 (4, 1, 128, 0, 64), (4, 1, 128, 50, 15), (8, 1, 64, 500, 12), (8, 1, 128, 500, 13),
                                                  (4, 1, 128, 1000, 24), (4, 1, 128, 1000, 25)])
 def test_planned_key_groups(rf, orc, stream, nh, nkv, hd, pos0, rows):
     _run(rf, orc, stream, nh, nkv, hd, pos0, rows, token_major=True)
