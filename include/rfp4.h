@@ -206,12 +206,16 @@ int mx4_quantize(rfp4_stream_t stream, uint64_t rows, uint64_t k, const void *sr
  * 16-byte aligned, scales 8-byte aligned.  The reference has only the
  * single m16n8k64 block-scaled tile (fp4_mma/src/main.rs:18-54) and its CPU
  * closed form D = sum_k A SFA B SFB (trackb/fp4_scale_test.cu:37); this is
- * that contraction at M x N x K.  Split-K shapes use a library workspace:
- * calls that overlap on one device race.  The tiled kernels (more than 32
- * activation rows) read the scales in a step-blocked layout (below), which
- * this entry point makes first in a library workspace of 64 MiB (one more
- * launch; shapes whose copies exceed it fail with RFP4_E_CAPACITY: use
- * fp4_gemm_tiled). */
+ * that contraction at M x N x K.  Up to 32 activation rows (K a multiple of
+ * 512, up to 16384), and from 33 to 64 rows of narrow matrices (K a multiple of
+ * 512, up to 8192; N at most 16 times the CUs), a few-row kernel reads the
+ * scales as they are.  Every other shape runs a tiled kernel, which reads them
+ * in a step-blocked layout (below) that this entry point makes first in a
+ * library workspace of 64 MiB (one more launch; shapes whose copies exceed it
+ * fail with RFP4_E_CAPACITY: use fp4_gemm_tiled), and may split K, with its
+ * partial sums in a library workspace: calls that overlap on one device race,
+ * on either.  Which shapes split can change between versions
+ * (rfp4_gemm_plan tells). */
 int fp4_gemm(rfp4_stream_t stream, uint32_t m, uint32_t n, uint32_t k, const uint8_t *a_codes,
              const uint8_t *a_scales, const uint8_t *w_codes, const uint8_t *w_scales, float *c);
 /* Step-blocked copy of [rows][k/32] E8M0 scales (k % 256 == 0): for each
@@ -235,7 +239,7 @@ int mx4_quantize_tiled(rfp4_stream_t stream, uint64_t rows, uint64_t k, const vo
  * mx4_scales_tile or mx4_quantize_tiled, or an engine's, see
  * llama_engine_weight_scales_tiled): no copy is made, so the call adds no
  * launch and has no workspace limit beyond fp4_gemm's split-K one.  The
- * few-row kernel (m <= 32) reads the row-major scales, the tiled kernels the
+ * few-row kernel (see fp4_gemm) reads the row-major scales, the tiled kernels the
  * step-blocked ones; both must describe the same scales.  Same results as
  * fp4_gemm, bit for bit.  No reference counterpart (see fp4_gemm). */
 int fp4_gemm_tiled(rfp4_stream_t stream, uint32_t m, uint32_t n, uint32_t k, const uint8_t *a_codes,

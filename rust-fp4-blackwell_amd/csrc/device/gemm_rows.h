@@ -191,17 +191,21 @@ RFP4_DEV void gemm_rows_body(const GemmArgs &g)
 // CU, the fragments strided over the grid's waves.  The activation rows
 // (16 MB x K/2 bytes) and their scales are brought into LDS once per
 // workgroup.  A wave holds the W bytes of a whole fragment in registers (4
-// loads per segment in flight, up to 32 KB per wave) and refills each
-// segment's registers with the next fragment's as soon as its MFMAs have read
-// them, so the stream does not drain between fragments and no wave waits for
-// another's partial sums.  A fragment's scales (16 rows x K/32 bytes) come in
+// loads per segment in flight, up to 32 KB per wave), needs no other wave's
+// partial sums, and where it takes more than one fragment (more than 8 per CU:
+// past 32768 rows on 256 CUs) refills each segment's registers with the next
+// one's as soon as its MFMAs have read them, so the stream does not drain
+// between fragments.  A fragment's scales (16 rows x K/32 bytes) come in
 // contiguous 16-byte chunks and are turned segment-major through 2 KB of LDS
 // of the wave's own (one chunk per lane and segment would touch every line of
 // them once per segment).  The sums are the K-split form's bit for bit: each
 // segment's 4 MFMAs start from zero and the segments are added in order.
 //
-// Bound by the W stream.  Codes as plain loads: the pattern (64 bytes of each
-// of 16 rows) reads 58.7 MB in 11.1 us, non-temporal in 12.5.  Against the
+// Bound by the W stream, and from 16 activation rows on by what follows it: at
+// 28672x4096 every wave has one fragment, and its activation reads, MFMAs and
+// stores come after the last of its loads (M = 1 13.4 us, M = 32 16.1).  Codes as
+// plain loads: the pattern (64 bytes of each of 16 rows) reads 58.7 MB in 11.1
+// us, non-temporal in 12.5.  Against the
 // K-split form at NF = 4 (8 waves, every load of the workgroup issued at once,
 // then MFMAs, LDS sums and stores with no load in flight), us at M = 32, 16, 1:
 // 28672x4096 18.5 -> 16.1, 16.2 -> 13.9, 14.0 -> 13.4; 20000x4096 17.3 ->

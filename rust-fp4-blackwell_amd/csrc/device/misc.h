@@ -111,7 +111,8 @@ RFP4_DEV void argmax_keys_body(const ArgmaxKeysArgs &a)
 // ---------------------------------------------------------------- end of decode step
 // Latency bound, a chain of dependent loads: the cursor and the prompt's next
 // token are fetched beside the keys, and every thread holds the token, so the
-// embedding row is the only load after the reduction (4008 keys: 5.4 -> 4.5 us).
+// embedding row is the only load after the reduction (4008 keys, in the trace
+// of the 8B step 5.8 -> 4.8 us).
 RFP4_DEV void step_body(const StepArgs &a)
 {
     const int pos = a.state->pos, step = a.state->step;

@@ -15,8 +15,9 @@
 // Bound by the latency of the gather: one 16-byte load and two float4 stores
 // per thread (k is a multiple of 256 here, so rows start 16-byte aligned), a
 // workgroup per 2048 elements of a row, so that a row takes one round trip
-// (one element per thread and trip before: 700 rows x 4096 12.9 us, now 9.3).
-// The ids are in pinned host memory: one load per workgroup.
+// (one element per thread and trip before).  The ids are in pinned host memory,
+// one load per workgroup: 700 rows x 4096 13.1 us, 10.0 with the ids on the
+// device, but then behind a copy that is a launch of its own.
 RFP4_DEV void embed_rows_body(const RowsArgs &a)
 {
     __shared__ uint32_t s_tok;

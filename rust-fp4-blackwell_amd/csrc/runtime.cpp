@@ -1251,7 +1251,12 @@ bool gemm_rows_has(int mb, int seg, int nf)
 }
 // W fragments per workgroup: the most (4, 2, 1) that still give three CUs in
 // four a workgroup (each workgroup shares its activation loads over its W
-// rows; measured above)
+// rows).  Measured (us, 1 / 2 / 4 fragments, K = 4096): 4096 rows at M = 32 6.5
+// / 7.4 / 8.8, 6144 rows 8.6 / 7.6 / 8.1, 12288 rows 12.0 / 12.0 / 9.9, 28672
+// rows 23.9 / 20.3 / 16.2.  The line between two and four dates from a kernel of
+// four fragments in K-split form; the wide form is already ahead at 10240 rows
+// (11.0 / 11.2 / 9.0) and, up to 16 activation rows, at 6144 (M = 16 7.4 / 6.8
+// / 5.9).
 int gemm_rows_nf(int mb, int seg, uint32_t n, uint32_t num_cus)
 {
     for (int nf = 4; nf > 1; nf /= 2)
@@ -1270,11 +1275,12 @@ uint32_t ceil_div(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); 
 // what the device shares.  Fitted to 21000 timings on MI355X (49
 // weight shapes of 512 .. 28672 rows and K 1024 .. 14336 at 8 to 2048
 // activation rows, and 413 random shapes; every compiled kernel, up to 8
-// splits, weights from HBM).  Past 32 rows the least estimate is within 1.2 %
-// (geometric mean; random shapes 1.9 %) of the fastest measured plan; the tile
-// thresholds used before were 18 % off it (2048x2048 at 48 rows split 8 ways
-// 9.9 us, 5.0 now; 11264x2048 at 320 rows 17.4, 9.7; 14336x4096 at 128 rows
-// 18.0, 12.5).
+// splits, weights from HBM).  On 2625 other random shapes (33 to 2048 rows, 512
+// to 28672 columns, K 1024 to 14336) the least estimate is 2.2 % (geometric
+// mean) off the fastest measured plan, and the tile thresholds used before 17 %.
+// It has no term for C rows that do not start on 64 bytes (N no multiple of 16),
+// which take up to twice as long to store: 256x256 tiles, 27564x1536 at 1254
+// rows 117 us, 26576x1536 at 1082 rows 56.
 struct GemmCost {
     int tile, nst;
     uint32_t occ;                 // workgroups per CU (registers and LDS of the compiled kernel)
@@ -1316,10 +1322,15 @@ bool gemm_kind_has(GemmKind kind, int tile, int nst)
 }
 
 // The cheapest tiled plan.  A forced tile or split (test hooks) is taken as it
-// is.  fp4_gemm covers the CUs (7/8 of them, 3/4 by tiles of 128x128 or more;
-// half with a short K or from 1024 rows on) by K splits where the splits fit
-// the workspace, and pads rows by at most a quarter; the prefill's projections
-// are free of that.
+// is.  The prefill's projections take the least estimate.  fp4_gemm and
+// fp4_gemm_tiled keep two promises of the thresholds they were planned by
+// before: they cover the CUs (7/8 of them, 3/4 by tiles of 128x128 or more; half
+// with a short K or from 1024 rows on) by K splits where the splits fit the
+// workspace, and pad rows by at most a quarter.  That costs them: on the 2625
+// shapes above their plans are 7.5 % off the fastest measured one (860x1024 at
+// 271 rows in four splits 8.4 us, unsplit 5.5; 9900x8960 at 43 rows 21.4,
+// without the padding rule 16.8), and 4 % of the shapes are more than 2 % slower
+// than by the thresholds (the most 1.25 times: 26576x1536 at 1082 rows).
 GemmPlan gemm_plan_tiles(uint32_t m, uint32_t n, uint32_t k, uint32_t cus, GemmKind kind)
 {
     const uint32_t nsuper = k / 256u;
@@ -1495,6 +1506,9 @@ int gemm_launch(hipStream_t stream, uint32_t m, uint32_t n, uint32_t k, const ui
         if (p.kz == 4u) {
             // a wave per fragment of 16 rows: one workgroup per CU, the waves
             // (at most 8) that spread the fragments evenly in the fewest rounds
+            // (us at M = 32, the rule's waves / one round more: 28672x4096 16.2
+            // / 16.0, 20000x4096 12.9 / 13.2, 14336x2048 6.6 / 7.0, 128256x4096
+            // 53.3 / 56.1)
             const uint32_t frags = ceil_div(n, 16u), cus = (uint32_t)rt->num_cus;
             waves = ceil_div(frags, cus * ceil_div(frags, 8u * cus));
             grid = std::min(ceil_div(frags, waves), cus);
